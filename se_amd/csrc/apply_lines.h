@@ -88,6 +88,82 @@ __device__ __forceinline__ int unk_line(int X, int M, int per, int off, int nU) 
     return (I >= 0 && I < nU) ? I : -1;
 }
 
+// Steps 1 and 3 for line t of element e, at column c and row r of a block s_u
+// with row pitch BW (line threads of any tile shape): the gradients along row
+// t and column t and their FP32 exchange; then, after a barrier, the line's
+// two sets of outputs, yx at the nodes (l, t) with the mass term and yy at
+// the nodes (t, l).
+template <int N>
+__device__ __forceinline__ void line_gradients(const OpParams& P, const double* s_u, int BW, int r, int c, int t,
+                                               int e, float* s_xf, float* s_ef, double (&uxi)[N + 1],
+                                               double (&uet)[N + 1]) {
+    constexpr int N1 = N + 1, NP = N1 * N1;
+    cdouble* Dc = (cdouble*)P.D;
+    double ur[N1], uc[N1];
+#pragma unroll
+    for (int k = 0; k < N1; k++) {
+        ur[k] = s_u[(r * N + t) * BW + c * N + k];
+        uc[k] = s_u[(r * N + k) * BW + c * N + t];
+    }
+#pragma unroll
+    for (int q = 0; q < N1; q++) {
+        double sx = 0.0, sy = 0.0;
+#pragma unroll
+        for (int k = 0; k < N1; k++) {
+            sx += Dc[q * N1 + k] * ur[k];
+            sy += Dc[q * N1 + k] * uc[k];
+        }
+        uxi[q] = sx;  // u_xi at (qx = q, qy = t)
+        uet[q] = sy;  // u_eta at (qx = t, qy = q)
+        __builtin_amdgcn_sched_barrier(0);  // one row of D live at a time
+    }
+#pragma unroll
+    for (int q = 0; q < N1; q++) {
+        s_xf[e * NP + q * N1 + t] = (float)uxi[q];  // [qx = q][qy = t]
+        s_ef[e * NP + q * N1 + t] = (float)uet[q];  // [qy = q][qx = t]
+    }
+}
+
+template <int N>
+__device__ __forceinline__ void line_outputs(const OpParams& P, const double* s_u, int BW, int r, int c, int t, int e,
+                                             const float* s_xf, const float* s_ef, const double* cf, const double* rf,
+                                             const float* cq, const float* rq, const double (&uxi)[N + 1],
+                                             const double (&uet)[N + 1], double (&yx)[N + 1], double (&yy)[N + 1]) {
+    constexpr int N1 = N + 1, NP = N1 * N1;
+    cdouble* DTc = (cdouble*)P.DT;
+    double fx[N1], fy[N1];
+    // row t (qy = t, qx = q): g01 = A2[q] QYw[t][q] + QXw[q][t] Y2w[t]
+    const double y0 = rf[t], y2w = rf[2 * N1 + t];
+#pragma unroll
+    for (int q = 0; q < N1; q++) {
+        const double ue = (double)s_ef[e * NP + t * N1 + q];  // u_eta at (q, t)
+        const double g01 = cf[2 * N1 + q] * (double)rq[t * N1 + q] + (double)cq[NP + t * N1 + q] * y2w;
+        fx[q] = cf[q] * y0 * uxi[q] + g01 * ue;
+    }
+    // column t (qx = t, qy = q): g01 = A2[t] QYw[q][t] + QXw[t][q] Y2w[q]
+    const double a1 = cf[N1 + t], a2 = cf[2 * N1 + t];
+#pragma unroll
+    for (int q = 0; q < N1; q++) {
+        const double ux = (double)s_xf[e * NP + t * N1 + q];  // u_xi at (t, q)
+        const double g01 = a2 * (double)rq[NP + t * N1 + q] + (double)cq[t * N1 + q] * rf[2 * N1 + q];
+        fy[q] = g01 * ux + a1 * rf[N1 + q] * uet[q];
+    }
+    const double my = rf[3 * N1 + t];
+#pragma unroll
+    for (int l = 0; l < N1; l++) {
+        double sx = 0.0, sy = 0.0;
+#pragma unroll
+        for (int q = 0; q < N1; q++) {
+            sx += DTc[l * N1 + q] * fx[q];
+            sy += DTc[l * N1 + q] * fy[q];
+        }
+        // node (l, t); the mass term re-reads u (fewer live registers)
+        yx[l] = sx + my * cf[3 * N1 + l] * s_u[(r * N + t) * BW + c * N + l];
+        yy[l] = sy;                                // node (t, l)
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
 template <int N, int MODE>
 __device__ __forceinline__ void apply_lines_tile(const OpParams& P, int tile,
                                                  const double* __restrict__ in, double* __restrict__ out,
@@ -118,8 +194,6 @@ __device__ __forceinline__ void apply_lines_tile(const OpParams& P, int tile,
     const bool halo_c = ex0 > 0 || P.per0, halo_r = ey0 > 0 || P.per1;
     const SE_GLOBAL double* gin = gview(in);
     SE_GLOBAL double* gout = gview(out);
-    cdouble* Dc = (cdouble*)P.D;
-    cdouble* DTc = (cdouble*)P.DT;
 
     // ---- 1. the tile's node block and its tables; two barriers ----------------
     for (int i = tid; i < BWU + BH; i += 256) {
@@ -177,71 +251,12 @@ __device__ __forceinline__ void apply_lines_tile(const OpParams& P, int tile,
     const int e = tid / N1, t = tid - (tid / N1) * N1;
     const int c = e % (TX + 1), r = e / (TX + 1);
     const bool live = e < NE && (c > 0 || halo_c) && (r > 0 || halo_r) && c <= txo && r <= tyo;
-    double uxi[N1], uet[N1];
-    if (live) {
-        double ur[N1], uc[N1];
-#pragma unroll
-        for (int k = 0; k < N1; k++) {
-            ur[k] = s_u[(r * N + t) * BW + c * N + k];
-            uc[k] = s_u[(r * N + k) * BW + c * N + t];
-        }
-#pragma unroll
-        for (int q = 0; q < N1; q++) {
-            double sx = 0.0, sy = 0.0;
-#pragma unroll
-            for (int k = 0; k < N1; k++) {
-                sx += Dc[q * N1 + k] * ur[k];
-                sy += Dc[q * N1 + k] * uc[k];
-            }
-            uxi[q] = sx;  // u_xi at (qx = q, qy = t)
-            uet[q] = sy;  // u_eta at (qx = t, qy = q)
-            __builtin_amdgcn_sched_barrier(0);  // one row of D live at a time
-        }
-#pragma unroll
-        for (int q = 0; q < N1; q++) {
-            s_xf[e * NP + q * N1 + t] = (float)uxi[q];  // [qx = q][qy = t]
-            s_ef[e * NP + q * N1 + t] = (float)uet[q];  // [qy = q][qx = t]
-        }
-    }
+    double uxi[N1], uet[N1], yx[N1], yy[N1];
+    if (live) line_gradients<N>(P, s_u, BW, r, c, t, e, s_xf, s_ef, uxi, uet);
     __syncthreads();
-    double yx[N1], yy[N1];
-    if (live) {
-        const double* cf = &s_cf[c * F];
-        const double* rf = &s_rf[r * F];
-        const float* cq = &s_cq[c * QS];
-        const float* rq = &s_rq[r * QS];
-        double fx[N1], fy[N1];
-        // row t (qy = t, qx = q): g01 = A2[q] QYw[t][q] + QXw[q][t] Y2w[t]
-        const double y0 = rf[t], y2w = rf[2 * N1 + t];
-#pragma unroll
-        for (int q = 0; q < N1; q++) {
-            const double ue = (double)s_ef[e * NP + t * N1 + q];  // u_eta at (q, t)
-            const double g01 = cf[2 * N1 + q] * (double)rq[t * N1 + q] + (double)cq[NP + t * N1 + q] * y2w;
-            fx[q] = cf[q] * y0 * uxi[q] + g01 * ue;
-        }
-        // column t (qx = t, qy = q): g01 = A2[t] QYw[q][t] + QXw[t][q] Y2w[q]
-        const double a1 = cf[N1 + t], a2 = cf[2 * N1 + t];
-#pragma unroll
-        for (int q = 0; q < N1; q++) {
-            const double ux = (double)s_xf[e * NP + t * N1 + q];  // u_xi at (t, q)
-            const double g01 = a2 * (double)rq[NP + t * N1 + q] + (double)cq[t * N1 + q] * rf[2 * N1 + q];
-            fy[q] = g01 * ux + a1 * rf[N1 + q] * uet[q];
-        }
-        const double my = rf[3 * N1 + t];
-#pragma unroll
-        for (int l = 0; l < N1; l++) {
-            double sx = 0.0, sy = 0.0;
-#pragma unroll
-            for (int q = 0; q < N1; q++) {
-                sx += DTc[l * N1 + q] * fx[q];
-                sy += DTc[l * N1 + q] * fy[q];
-            }
-            // node (l, t); the mass term re-reads u (fewer live registers)
-            yx[l] = sx + my * cf[3 * N1 + l] * s_u[(r * N + t) * BW + c * N + l];
-            yy[l] = sy;                                // node (t, l)
-            __builtin_amdgcn_sched_barrier(0);
-        }
-    }
+    if (live)
+        line_outputs<N>(P, s_u, BW, r, c, t, e, s_xf, s_ef, &s_cf[c * F], &s_rf[r * F], &s_cq[c * QS], &s_rq[r * QS],
+                        uxi, uet, yx, yy);
     __syncthreads();  // the exchange arrays are read; s_o takes the outputs
     if (live) {
 #pragma unroll

@@ -782,6 +782,10 @@ int pcg_fp64(se_op* op, const double* d_f, double* d_x, const se_solve_opts& o, 
         hipLaunchKernelGGL(k_scale_copy, dim3(vb), dim3(kBlock), 0, s, n, (double)op->sign, op->dinv.as<double>(),
                            op->dinv_s.as<double>());
     }
+    if (!op->h_state) SE_HIP(hipHostMalloc(&op->h_state, sizeof(CgState), hipHostMallocDefault));
+    bool done = false;
+    rc = pcg_grid(op, d_f, d_x, o, info, done);
+    if (rc || done) return rc;
     CgState h{};
     h.maxit = std::max(o.maxit, 0);
     h.null_space = o.null_space ? 1 : 0;
@@ -794,7 +798,6 @@ int pcg_fp64(se_op* op, const double* d_f, double* d_x, const se_solve_opts& o, 
         if (rc) return rc;
     }
     double* dh = o.history ? d_hist.as<double>() : nullptr;
-    if (!op->h_state) SE_HIP(hipHostMalloc(&op->h_state, sizeof(CgState), hipHostMallocDefault));
     CgState* hs = (CgState*)op->h_state;
     SE_HIP(hipEventRecord(c->ev0, s));
     *hs = h;  // uploads go through the pinned host copy

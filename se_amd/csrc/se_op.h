@@ -33,6 +33,9 @@ struct se_op {
     void* h_state = nullptr;
     hipGraphExec_t graph_exec = nullptr;
     int graph_iters = 0;
+    se::DevBuf grid_slots, grid_work;        // one-launch solve (pcg_grid.hip): sum slots, work
+    bool grid_dirty = false;                 // they need clearing first
+    int grid_turn = 0;                       // the region the next solve uses
     hipGraphExec_t graph_exec_lo = nullptr;
     int graph_iters_lo = 0;
     // spectral vanishing viscosity term (svv.hip): dt, cutoff (0: none), the
@@ -47,7 +50,7 @@ struct se_op {
         se::fdm_release(this);
         se::DevBuf* bufs[] = {&sep, &sep_state, &sep_part, &dinv, &dinv_s, &lift, &tabs, &qtabs, &state, &partials, &b, &x, &r, &p, &q, &f,
                               &sx, &sy, &sfield, &sfield2, &lo_r, &lo_p, &lo_q, &lo_z, &lo_x, &lo_dinv,
-                              &lo_geo, &d64, &svv_mk};
+                              &lo_geo, &d64, &svv_mk, &grid_slots, &grid_work};
         for (auto* b : bufs) b->release();
         if (graph_exec_lo) (void)hipGraphExecDestroy(graph_exec_lo);
         graph_exec_lo = nullptr;
@@ -61,6 +64,7 @@ OpParams op_params(const se_op* op, double scale);
 int op_apply_dev(se_op* op, const double* d_x, double* d_y, double scale, bool dot);
 int op_ensure_work(se_op* op);
 int pcg_fp64(se_op* op, const double* d_f, double* d_x, const se_solve_opts& o, se_solve_info& info);
+int pcg_grid(se_op* op, const double* d_f, double* d_x, const se_solve_opts& o, se_solve_info& info, bool& done);
 int pcg_mixed(se_op* op, const double* d_f, double* d_x, const se_solve_opts& o, se_solve_info& info);
 // FDM-preconditioned CG (fdm.hip); solve_pc resolves SE_PC_DEFAULT
 int pcg_fdm(se_op* op, const double* d_f, double* d_x, const se_solve_opts& o, se_solve_info& info);
