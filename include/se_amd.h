@@ -52,8 +52,10 @@ enum { SE_DETJ_LITERAL = 0, SE_DETJ_PHYSICAL = 1 };
  * whose residual, norms and update are FP64.  FP64_FP32C / FP64_BF16C (FDM
  * preconditioner only): FP64 CG whose preconditioner's first application --
  * the one that sets the residual's floor -- runs in FP64 and later ones,
- * corrections of the residual it left, in FP32, resp. with BF16 operands
- * (which, like BF16_IR, may stagnate on a near-singular system). */
+ * corrections of the residual it left, may run in FP32, resp. with BF16
+ * operands.  These are the least precisions: FDM transforms of lines of up to
+ * 256 elements run in FP64 in every one of them but BF16_IR (their plane-wave
+ * form is faster there than dense transforms of fewer bits). */
 enum { SE_PREC_FP64 = 0, SE_PREC_FP32_IR = 1, SE_PREC_BF16_IR = 2, SE_PREC_FP64_FP32C = 3, SE_PREC_FP64_BF16C = 4 };
 
 /* Preconditioner.  JACOBI: the reference's (PETSc -pc_type jacobi; FP64) or

@@ -43,8 +43,10 @@
 #include "apply_kernels.h"
 #include "apply_lines.h"
 #include "fdm_host.h"
+#include "fdm_wave.h"
 #include "se_common.h"
 #include "se_op.h"
+#include "wave_host.h"
 
 namespace se {
 
@@ -391,7 +393,7 @@ struct FbMember {
     const double* f;
     double *b, *x, *r, *p, *q, *z;
     double* pv;  // [nch]      r.r after start / update / restart
-    double* pz;  // [3][ntz]   FDM partials r.z, sum z, sum r
+    double* pz;  // [ntr] FDM partials of r.z, then [2][ntz] of sum z, sum r
     double* pa;  // [nap]      p.q
     double* pt;  // [2][nap]   sum t, sum t^2 of the true residual
     double* ps;  // [nch]      sum of sgn f
@@ -399,7 +401,8 @@ struct FbMember {
     void* rp;    //            r in the transforms' type T, padded: pass 1's operand
     void* rpc;   //            the same for the corrections' transforms (after an update)
     CgState* st;
-    int n, nch, ntz, null_space;
+    int n, nch, ntr, ntz, null_space;
+    int wave;   // wave-form transforms: they read r itself, nothing is packed
     int fused;  // p.q and the true residual from the apply's epilogue (no SVV term)
     int nap;    // partials of p.q and of the true residual: apply tiles (fused), else nch
     int nU0, nP0, rprec;  //   unknown-grid row length, padded row length, T (FDM_F64 / F32 / BF16)
@@ -410,6 +413,7 @@ struct FbMember {
 // r[i] into the packed residual (row i / nU0, column i mod nU0), rounded to T
 // as the pack kernel rounds it
 __device__ __forceinline__ void put_packed_to(const FbMember& M, void* rp, int prec, int i, double v) {
+    if (M.wave) return;
     const int J = i / M.nU0, I = i - J * M.nU0;
     const size_t k = (size_t)J * M.nP0 + I;
     if (prec == FDM_F64) ((SE_GLOBAL double*)rp)[k] = v;
@@ -489,7 +493,12 @@ __global__ __launch_bounds__(FB_NT) void k_fb_dir(const FbMember* __restrict__ M
         double tr[1], tz[3];
         reduce_partials<1, FB_NT>(M.pv, M.nch, tr);  // (its barriers publish s_stop)
         if (s_stop) continue;
-        reduce_partials<3, FB_NT>(M.pz, M.ntz, tz);
+        {
+            double t1[1], t2[2] = {0.0, 0.0};
+            reduce_partials<1, FB_NT>(M.pz, M.ntr, t1);
+            if (M.null_space) reduce_partials<2, FB_NT>(M.pz + M.ntr, M.ntz, t2);
+            tz[0] = t1[0], tz[1] = t2[0], tz[2] = t2[1];
+        }
         const double rr = tr[0];
         const bool finite = (rr - rr == 0.0) && (tz[0] - tz[0] == 0.0);
         const double mu = M.null_space ? tz[1] / M.n : 0.0;
@@ -724,7 +733,23 @@ struct VMats {
     DevBuf v, vT;
 };
 
+// A line's wave-form tables on the device (wave_host.h, fdm_wave.h), shared by
+// the operators of the same line.
+struct WaveLineDev {
+    se_wave::Line L;
+    DevBuf tiles;  // WaveTile: nf forward, then nb backward
+    int kf = 0, kb = 0, nf = 0, nb = 0;
+    DevBuf fwd, bwd, phi;
+};
+
 struct FdmOp {
+    // the wave form (every precision but BF16 operands; lines of up to
+    // se_wave::kMaxE elements): tables per direction, and by mode
+    bool wave = false;
+    std::shared_ptr<const WaveLineDev> wx, wy;
+    DevBuf wlx, wex, wly, wey, wt1;
+    double wdtol = 0.0;
+    bool dense = false;       // the members below up to `prec` are built
     FdmPlan* self = nullptr;  // the one-member plan of this operator's own solves
     int nU0 = 0, nU1 = 0, nP0 = 0, nP1 = 0;
     double dtol = 0.0;
@@ -749,6 +774,108 @@ void fdm_release(se_op* op) {
 }
 
 namespace {
+
+// wave-form lines shared by operators of the same line on one device (keyed by
+// the element's tables); a line nobody uses any more is dropped
+std::mutex g_wave_mu;
+std::map<std::string, std::weak_ptr<const WaveLineDev>> g_wave_cache;
+
+// axis of op's mesh: the wave form of its line; null if the line has none.
+// The element tables are the mean over the elements (equal up to round-off on
+// the uniform mesh).
+int wave_line_of(const se_op* op, int axis, std::shared_ptr<const WaveLineDev>& out) {
+    const se_mesh* m = op->mesh;
+    const int N = m->N, n1 = N + 1, CS = 4 * n1 + n1 * n1, ne = m->nEls[axis], per = m->periodic[axis];
+    const int lo = per ? 0 : (axis == 0 ? m->bc[2] : m->bc[0]), hi = per ? 0 : (axis == 0 ? m->bc[3] : m->bc[1]);
+    const size_t base = axis == 0 ? 0 : (size_t)m->nEls[0] * CS;
+    std::vector<double> P(n1, 0.0), S(n1, 0.0);
+    const double sgn = (double)op->sign;
+    for (int e = 0; e < ne; e++) {
+        const double* T = &op->tabs_host[base + (size_t)e * CS];
+        for (int q = 0; q < n1; q++) {
+            P[q] += (axis == 0 ? T[q] : T[n1 + q]) / ne;
+            S[q] += sgn * op->c_lap * (axis == 0 ? T[n1 + q] : T[q]) / ne;
+        }
+    }
+    for (double v : S)
+        if (!(v > 0.0)) return SE_OK;
+    std::string key((const char*)P.data(), sizeof(double) * n1);
+    key.append((const char*)S.data(), sizeof(double) * n1);
+    const int k[6] = {m->ctx->device, ne, N, per, lo, hi};
+    key.append((const char*)k, sizeof(k));
+    std::lock_guard<std::mutex> lk(g_wave_mu);
+    auto it = g_wave_cache.find(key);
+    if (it != g_wave_cache.end() && (out = it->second.lock())) return SE_OK;
+    for (auto i = g_wave_cache.begin(); i != g_wave_cache.end();)
+        i = i->second.expired() ? g_wave_cache.erase(i) : std::next(i);
+    const std::vector<double>& D = m->gll.D;
+    std::vector<double> K((size_t)n1 * n1, 0.0);
+    for (int a = 0; a < n1; a++)
+        for (int b = 0; b < n1; b++)
+            for (int q = 0; q < n1; q++) K[a * n1 + b] += D[q * n1 + a] * P[q] * D[q * n1 + b];
+    auto w = std::make_shared<WaveLineDev>();
+    if (!se_wave::wave_line(ne, N, per != 0, lo != 0, hi != 0, K, S, w->L)) return SE_OK;
+    const se_wave::Line& L = w->L;
+    SE_CHECK(L.n == m->nU[axis], SE_ERR_STATE, "FDM: the line's unknowns are not the mesh's");
+    // operand order, per block [row tile][k step][lane], lane l: row l & 15, k l >> 4
+    const int E = L.E, E16 = L.E16;
+    std::vector<double> f, b;
+    for (const auto& k : L.blk) {
+        w->kf = std::max(w->kf, 2 * ((k.nk + 7) / 8));
+        w->kb = std::max(w->kb, 2 * ((k.np + 7) / 8));
+    }
+    const int R = 1 << wave_log_r(L.E);
+    std::vector<WaveTile> tf, tb;
+    for (int kd = 0; kd < 6; kd++) {
+        const auto& k = L.blk[kd];
+        const int kind = kd / 2, parts = kind == 0 ? 1 : (kind == 1 ? L.nS : L.nA);
+        if (k.nk == 0 || k.np == 0 || parts == 0) continue;
+        auto wave = [&](int slot, int phase) {
+            return slot < k.nk && phase < k.np ? L.F[kind][(size_t)(k.s0 + slot) * E16 + (k.b0 + phase) % E] : 0.0;
+        };
+        for (int fwd = 1; fwd >= 0; fwd--) {
+            const int rows = fwd ? k.np : k.nk, KS = fwd ? w->kf : w->kb;
+            std::vector<double>& o = fwd ? f : b;
+            for (int mt = 0; mt < (rows + 15) / 16; mt++) {
+                WaveTile t;
+                t.of = (int)o.size();
+                t.row = 16 * mt;
+                t.at = kd & 1 ? k.top : 0;
+                t.step = kd & 1 ? -1 : 1;
+                t.b0 = k.b0;
+                t.cnt = rows;
+                for (int c = 0; c < parts * R; c += 16) {
+                    t.col = (kind == 0 ? 0 : (kind == 1 ? R : R * (1 + L.nS))) + c;
+                    t.w = std::min(16, parts * R - c);
+                    (fwd ? tf : tb).push_back(t);
+                }
+                for (int ks = 0; ks < KS; ks++)
+                    for (int l = 0; l < 64; l++) {
+                        const int m = 16 * mt + (l & 15), kk = 4 * ks + (l >> 4);
+                        o.push_back(fwd ? wave(kk, m) : wave(m, kk));
+                    }
+            }
+        }
+    }
+    w->nf = (int)tf.size();
+    w->nb = (int)tb.size();
+    SE_CHECK(std::max(w->nf, w->nb) <= 8 * (wave_long(E) ? 7 : 4), SE_ERR_STATE, "FDM: too many tiles for a line");
+    tf.insert(tf.end(), tb.begin(), tb.end());
+    auto up = [&](DevBuf& d, const void* src, size_t nb) -> int {
+        int rc = d.alloc(nb);
+        if (rc) return rc;
+        SE_HIP(hipMemcpy(d.ptr, src, nb, hipMemcpyHostToDevice));
+        return SE_OK;
+    };
+    int rc = up(w->fwd, f.data(), sizeof(double) * f.size());
+    if (!rc) rc = up(w->bwd, b.data(), sizeof(double) * b.size());
+    if (!rc) rc = up(w->tiles, tf.data(), sizeof(WaveTile) * tf.size());
+    if (!rc) rc = up(w->phi, L.phi.data(), sizeof(double) * L.phi.size());
+    if (rc) return rc;
+    g_wave_cache[key] = w;
+    out = w;
+    return SE_OK;
+}
 
 // eigen-decompositions of (G, S) shared by operators of the same line
 // (keyed by the exact bytes of G and S)
@@ -835,7 +962,138 @@ int vmats_of(const std::shared_ptr<const se_fdm::Fdm1D>& e, int nP, int prec, in
     return SE_OK;
 }
 
+// the modes of op in the wave form: eigenvalues, mass factors (the operators
+// of one line differ in c_mass) and the transforms' intermediate
+int wave_modes_prepare(se_op* op, FdmOp* F) {
+    const se_mesh* m = op->mesh;
+    const int N = m->N, n1 = N + 1, CS = 4 * n1 + n1 * n1;
+    const double sgn = (double)op->sign;
+    double lmax[2] = {0.0, 0.0}, emax[2] = {0.0, 0.0};
+    for (int axis = 0; axis < 2; axis++) {
+        const se_wave::Line& L = axis == 0 ? F->wx->L : F->wy->L;
+        const int ne = m->nEls[axis];
+        const size_t base = axis == 0 ? 0 : (size_t)m->nEls[0] * CS;
+        std::vector<double> M(n1, 0.0);
+        for (int e = 0; e < ne; e++)
+            for (int q = 0; q < n1; q++)
+                M[q] += (axis == 0 ? sgn * op->c_mass : 1.0) * op->tabs_host[base + (size_t)e * CS + 3 * n1 + q] / ne;
+        const size_t cnt = (size_t)L.E * N;
+        std::vector<double> lam(cnt + 16, 1.0), em(cnt + 16, 0.0);  // (the kernels read up to a block past the end)
+        for (int c = 0; c < L.E; c++)
+            for (int j = 0; j < N; j++) {
+                const size_t k = (size_t)c * N + j;
+                lam[k] = L.lambda[k];
+                if (!L.have[k]) continue;
+                for (int t = 0; t < N; t++) {
+                    const double f = L.phi[((size_t)t * N + j) * L.E16 + c];
+                    const int i = t <= L.nS ? t : t - L.nS;
+                    em[k] += f * f * (t == 0 ? M[0] + M[N] : 0.5 * (M[i] + M[N - i]));
+                }
+                lmax[axis] = std::max(lmax[axis], std::fabs(lam[k]));
+                emax[axis] = std::max(emax[axis], std::fabs(em[k]));
+            }
+        DevBuf &dl = axis == 0 ? F->wlx : F->wly, &de = axis == 0 ? F->wex : F->wey;
+        int rc = dl.alloc(sizeof(double) * lam.size());
+        if (!rc) rc = de.alloc(sizeof(double) * em.size());
+        if (rc) return rc;
+        SE_HIP(hipMemcpy(dl.ptr, lam.data(), sizeof(double) * lam.size(), hipMemcpyHostToDevice));
+        SE_HIP(hipMemcpy(de.ptr, em.data(), sizeof(double) * em.size(), hipMemcpyHostToDevice));
+    }
+    // a mode whose D is this small is the constant null mode of a singular
+    // (periodic / Neumann Poisson) operator
+    F->wdtol = 1e-11 * (lmax[0] + lmax[1] + emax[0] * emax[1]);
+    const se_wave::Line& X = F->wx->L;
+    const int R = 1 << wave_log_r(X.E);
+    return F->wt1.alloc(sizeof(double) * (size_t)X.E * N * ((F->nU1 + R - 1) / R * R));
+}
+
+// op's transforms in this precision take the wave form: always where the line
+// has one -- FP64 waves beat the dense transforms with FP32 or BF16 operands
+// too, which also need more iterations (solves, dense -> waves: 1024 x 1024
+// unknowns in FP64 589 -> 356 us; 225 x 145 in FP32 231 -> 120 us; 24 ragged
+// channels in FP32 586 -> 325 us; the 512-member ensemble with BF16 corrections
+// 3536 -> 3164 us) -- except for BF16 operands throughout, whose rounding is
+// what the caller asks for.
+bool fdm_wave(const se_op* op, int prec) { return op->fdm->wave && prec != FDM_BF16; }
+
 }  // namespace
+
+int wave_blocks(const se_op* op, int mode) {  // workgroups of WAVE_X / WAVE_XB, of WAVE_Y
+    const se_wave::Line &X = op->fdm->wx->L, &Y = op->fdm->wy->L;
+    const int lines = mode == WAVE_Y ? X.E * X.N : op->fdm->nU1, lg = wave_log_r(mode == WAVE_Y ? Y.E : X.E);
+    return (lines + (1 << lg) - 1) >> lg;
+}
+// z = FDM(r) of op in the wave form
+WaveTask wave_task(const se_op* op, const double* r, double* z, double* part, int null_space) {
+    const FdmOp* F = op->fdm;
+    WaveTask t{};
+    auto dim = [&](const WaveLineDev& w) {
+        WaveDim d;
+        d.fwd = w.fwd.as<double>();
+        d.bwd = w.bwd.as<double>();
+        d.phi = w.phi.as<double>();
+        d.ne = w.L.ne;
+        d.off = w.L.off;
+        d.vs = w.L.vs;
+        d.mirror = w.L.mirror[0] >= 0;
+        d.kf = w.kf;
+        d.kb = w.kb;
+        d.n0 = w.L.blk[0].nk;
+        d.n1 = w.L.blk[2].nk;
+        d.tf = w.tiles.as<WaveTile>();
+        d.tb = d.tf + w.nf;
+        d.nf = w.nf;
+        d.nb = w.nb;
+        d.n = w.L.n;
+        d.E = w.L.E;
+        d.E16 = w.L.E16;
+        d.logR = wave_log_r(w.L.E);
+        d.LD = wave_ld(w.L.N, d.logR);
+        return d;
+    };
+    t.x = dim(*F->wx);
+    t.y = dim(*F->wy);
+    t.N = F->wx->L.N;
+    t.nS = F->wx->L.nS;
+    t.nA = F->wx->L.nA;
+    t.t1 = F->wt1.as<double>();
+    t.r = r;
+    t.z = z;
+    t.part_rz = part;
+    t.part_zr = part + wave_blocks(op, WAVE_Y);
+    t.null_space = null_space;
+    t.lx = F->wlx.as<double>();
+    t.ly = F->wly.as<double>();
+    t.ex = F->wex.as<double>();
+    t.ey = F->wey.as<double>();
+    t.dtol = F->wdtol;
+    return t;
+}
+size_t wave_lds_of(const se_op* op, int mode) {
+    const se_wave::Line& L = mode == WAVE_Y ? op->fdm->wy->L : op->fdm->wx->L;
+    return wave_lds(L.N, L.E, L.E16, wave_ld(L.N, wave_log_r(L.E)));
+}
+// multiply-adds of one direction's transform, times 2
+double wave_flops(const se_op* op, int axis) {
+    const FdmOp* F = op->fdm;
+    const se_wave::Line& L = axis == 0 ? F->wx->L : F->wy->L;
+    return 2.0 * F->nU0 * F->nU1 * ((L.mirror[0] >= 0 ? 0.5 : 1.0) * L.E + L.N);
+}
+
+int launch_wave(int mode, bool lng, const WaveTask* tasks, const int2* work, int nwork, size_t lds, hipStream_t s,
+                int skip, int to_p) {
+    if (nwork <= 0) return SE_OK;
+    auto go = [&](auto k) -> int {
+        if (lds > 64 * 1024)
+            SE_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                       (int)lds));
+        hipLaunchKernelGGL(k, dim3(nwork), dim3(kWaveT), lds, s, tasks, work, nwork, skip, to_p);
+        return SE_OK;
+    };
+    if (mode == WAVE_X) return lng ? go(k_fdm_wave<WAVE_X, true>) : go(k_fdm_wave<WAVE_X, false>);
+    if (mode == WAVE_Y) return lng ? go(k_fdm_wave<WAVE_Y, true>) : go(k_fdm_wave<WAVE_Y, false>);
+    return lng ? go(k_fdm_wave<WAVE_XB, true>) : go(k_fdm_wave<WAVE_XB, false>);
+}
 
 // FDM tables of op (FP64 part: eigenvectors, eigenvalues, mass factors and
 // work vectors) and the transforms in precision `prec`
@@ -853,6 +1111,40 @@ int fdm_prepare(se_op* op, int prec) {
     if (rc) return rc;
     if (!op->fdm) {
         std::unique_ptr<FdmOp> F(new FdmOp);
+        F->nU0 = m->nU[0];
+        F->nU1 = m->nU[1];
+        F->nP0 = pad64(F->nU0);
+        F->nP1 = pad64(F->nU1);
+        rc = wave_line_of(op, 0, F->wx);
+        if (!rc) rc = wave_line_of(op, 1, F->wy);
+        if (rc) return rc;
+        F->wave = F->wx && F->wy;
+        int pz = 3 * (F->nP1 / 64) * (F->nP0 / 64);
+        if (F->wave) {
+            rc = wave_modes_prepare(op, F.get());
+            if (rc) return rc;
+            const int Rx = 1 << wave_log_r(F->wx->L.E);
+            const int Ry = 1 << wave_log_r(F->wy->L.E);
+            pz = std::max(pz, 2 * ((F->nU1 + Rx - 1) / Rx) + (F->wx->L.E * m->N + Ry - 1) / Ry);
+        }
+        const int n = std::max(m->n, 1);
+        const int nch = (n + FB_CH - 1) / FB_CH;
+        rc = F->z.alloc(sizeof(double) * n);
+        if (!rc) rc = F->pv.alloc(sizeof(double) * nch);
+        // p.q and true-residual partials: per chunk, or per apply tile when
+        // the applies form them
+        const int nap = std::max(nch, line_tiles(m->N, m->nEls[0], m->nEls[1]));
+        if (!rc) rc = F->pa.alloc(sizeof(double) * nap);
+        if (!rc) rc = F->ps.alloc(sizeof(double) * nch);
+        if (!rc) rc = F->pt.alloc(sizeof(double) * 2 * nap);
+        if (!rc) rc = F->pz.alloc(sizeof(double) * pz);
+        if (!rc) rc = F->st.alloc(sizeof(CgState));
+        if (rc) return rc;
+        op->fdm = F.release();
+    }
+    if (fdm_wave(op, prec)) return SE_OK;
+    FdmOp* F = op->fdm;
+    if (!F->dense) {
         const int N = m->N;
         std::vector<double> gx, X0, X1, MX, gy, Y0, Y1, MY;
         assemble_line(m, op, 0, gx, X0, X1, MX);
@@ -871,10 +1163,6 @@ int fdm_prepare(se_op* op, int prec) {
         F->ex1 = eig_1d(m->nU[0], N, m->periodic[0], gx, sx);
         F->ey1 = eig_1d(m->nU[1], N, m->periodic[1], gy, sy);
         SE_CHECK(F->ex1 && F->ey1, SE_ERR_STATE, "FDM preconditioner: 1-D eigenproblem failed");
-        F->nU0 = m->nU[0];
-        F->nU1 = m->nU[1];
-        F->nP0 = pad64(F->nU0);
-        F->nP1 = pad64(F->nU1);
         const se_fdm::Fdm1D &Ex = *F->ex1, &Ey = *F->ey1;
         std::vector<double> lx(F->nP0, 0.0), ex(F->nP0, 0.0), ly(F->nP1, 0.0), ey(F->nP1, 0.0);
         double lmax = 0.0, emx = 0.0, emy = 0.0;
@@ -907,23 +1195,8 @@ int fdm_prepare(se_op* op, int prec) {
         SE_HIP(hipMemcpy(F->ex.ptr, ex.data(), sizeof(double) * F->nP0, hipMemcpyHostToDevice));
         SE_HIP(hipMemcpy(F->ly.ptr, ly.data(), sizeof(double) * F->nP1, hipMemcpyHostToDevice));
         SE_HIP(hipMemcpy(F->ey.ptr, ey.data(), sizeof(double) * F->nP1, hipMemcpyHostToDevice));
-        const int n = std::max(m->n, 1);
-        const int nch = (n + FB_CH - 1) / FB_CH;
-        const int ntz = (F->nP1 / 64) * (F->nP0 / 64);
-        rc = F->z.alloc(sizeof(double) * n);
-        if (!rc) rc = F->pv.alloc(sizeof(double) * nch);
-        // p.q and true-residual partials: per chunk, or per apply tile when
-        // the applies form them
-        const int nap = std::max(nch, line_tiles(m->N, m->nEls[0], m->nEls[1]));
-        if (!rc) rc = F->pa.alloc(sizeof(double) * nap);
-        if (!rc) rc = F->ps.alloc(sizeof(double) * nch);
-        if (!rc) rc = F->pt.alloc(sizeof(double) * 2 * nap);
-        if (!rc) rc = F->pz.alloc(sizeof(double) * 3 * ntz);
-        if (!rc) rc = F->st.alloc(sizeof(CgState));
-        if (rc) return rc;
-        op->fdm = F.release();
+        F->dense = true;
     }
-    FdmOp* F = op->fdm;
     FdmOp::Prec& P = F->prec[prec];
     if (!P.ready) {
         const int dev = m->ctx->device;
@@ -1066,6 +1339,8 @@ struct FdmPlan {
     int prec = -1, cprec = -1;  // the transforms' precision: first application, corrections
     DevBuf d_members, d_tasks;  // FbMember[count], GemmTask[4 count]
     DevBuf d_tasks_c;           // GemmTask[4 count] of the corrections (cprec != prec)
+    DevBuf d_wtasks;            // WaveTask[count]; of a wave-form member the GemmTasks are unused
+    std::vector<WaveTask> h_wtasks;
     std::vector<FbMember> h_members;
     // FP64 apply descriptors per order (p -> q and x -> q)
     struct Order {
@@ -1090,9 +1365,10 @@ struct FdmPlan {
     struct Lists {
         std::vector<char> on;  // the member flags these lists were built for
         DevBuf d;
-        const int2 *vwork = nullptr, *gwork = nullptr, *apply[7] = {};
+        const int2 *vwork = nullptr, *gwork = nullptr, *wave[4] = {}, *apply[7] = {};
         const int* list = nullptr;
-        int n_vwork = 0, n_gwork = 0, n_apply[7] = {}, n_list = 0;
+        int n_vwork = 0, n_gwork = 0, n_wave[4] = {}, n_apply[7] = {}, n_list = 0;
+        size_t lds[4] = {};  // wave lists: x lines, long x lines, y, long y; the largest line block of each
         unsigned long long used = 0;
     };
     static constexpr int kListCache = 8;
@@ -1253,7 +1529,7 @@ void xcd_order(const FdmPlan* pl, const std::vector<char>& on, std::vector<int2>
     std::vector<double> cost;
     std::vector<const void*> cls;
     for (int i = 0; i < (int)pl->ops.size(); i++) {
-        if (!on[i]) continue;
+        if (!on[i] || pl->h_members[i].wave) continue;
         const FdmOp* F = pl->ops[i]->fdm;
         ids.push_back(i);
         tiles.push_back(pl->h_members[i].ntz);
@@ -1261,6 +1537,27 @@ void xcd_order(const FdmPlan* pl, const std::vector<char>& on, std::vector<int2>
         cls.push_back(F->ex1.get());
     }
     xcd_interleave(ids, tiles, cost, cls, out);
+}
+
+// wave list `which` (blocks of x lines, of long x lines, of y lines, long y lines)
+size_t wave_order(const FdmPlan* pl, const std::vector<char>& on, int which, std::vector<int2>& out) {
+    const int mode = which >= 2 ? WAVE_Y : WAVE_X;
+    std::vector<int> ids, tiles;
+    std::vector<double> cost;
+    std::vector<const void*> cls;
+    size_t lds = 0;
+    for (int i = 0; i < (int)pl->ops.size(); i++) {
+        if (!on[i] || !pl->h_members[i].wave) continue;
+        const FdmOp* F = pl->ops[i]->fdm;
+        if (wave_long((mode == WAVE_Y ? F->wy : F->wx)->L.E) != (which % 2 == 1)) continue;
+        ids.push_back(i);
+        tiles.push_back(wave_blocks(pl->ops[i], mode));
+        cost.push_back(wave_flops(pl->ops[i], mode == WAVE_Y ? 1 : 0));
+        cls.push_back(mode == WAVE_Y ? F->wy.get() : F->wx.get());
+        lds = std::max(lds, wave_lds_of(pl->ops[i], mode));
+    }
+    xcd_interleave(ids, tiles, cost, cls, out);
+    return lds;
 }
 
 // list set `set` switched to the members flagged in `on`: their lists from
@@ -1274,7 +1571,7 @@ int plan_lists(FdmPlan* pl, int set, const std::vector<char>& on, hipStream_t s)
             S.cur = e.get();
             return SE_OK;
         }
-    std::vector<int2> vwork, gwork, apply[7];
+    std::vector<int2> vwork, gwork, wave[4], apply[7];
     std::vector<int> list;
     for (int i = 0; i < (int)pl->ops.size(); i++) {
         if (!on[i]) continue;
@@ -1282,6 +1579,8 @@ int plan_lists(FdmPlan* pl, int set, const std::vector<char>& on, hipStream_t s)
         for (int c = 0; c < pl->h_members[i].nch; c++) vwork.push_back(make_int2(i, c));
     }
     xcd_order(pl, on, gwork);
+    size_t lds[4];
+    for (int k = 0; k < 4; k++) lds[k] = wave_order(pl, on, k, wave[k]);
     for (int k = 0; k < (int)pl->orders.size(); k++) {
         const FdmPlan::Order& o = pl->orders[k];
         std::vector<int> ids, tiles;
@@ -1300,6 +1599,7 @@ int plan_lists(FdmPlan* pl, int set, const std::vector<char>& on, hipStream_t s)
     }
     // packed: vector items, transform items, per-order apply items (int2), member list (int)
     size_t n2 = vwork.size() + gwork.size();
+    for (const auto& w : wave) n2 += w.size();
     for (const auto& a : apply) n2 += a.size();
     const size_t bytes = sizeof(int2) * n2 + sizeof(int) * list.size();
     if (bytes > S.hcap) {
@@ -1333,6 +1633,11 @@ int plan_lists(FdmPlan* pl, int set, const std::vector<char>& on, hipStream_t s)
     };
     L->vwork = reinterpret_cast<const int2*>(put(vwork.data(), sizeof(int2) * vwork.size()));
     L->gwork = reinterpret_cast<const int2*>(put(gwork.data(), sizeof(int2) * gwork.size()));
+    for (int k = 0; k < 4; k++) {
+        L->wave[k] = reinterpret_cast<const int2*>(put(wave[k].data(), sizeof(int2) * wave[k].size()));
+        L->n_wave[k] = (int)wave[k].size();
+        L->lds[k] = lds[k];
+    }
     for (int k = 0; k < 7; k++) {
         L->apply[k] = reinterpret_cast<const int2*>(put(apply[k].data(), sizeof(int2) * apply[k].size()));
         L->n_apply[k] = (int)apply[k].size();
@@ -1361,11 +1666,25 @@ int plan_pass(FdmPlan* pl, int set, int pass, hipStream_t s, int skip = 0, int t
                        L.n_gwork, s, skip, false, pass == 3 ? to_p : FDM_TO_Z);
 }
 
-// z = FDM(r) of the listed members: four passes
+// one kernel of the listed wave-form members' transforms
+int plan_wave(FdmPlan* pl, int set, int mode, hipStream_t s, int skip = 0, int to_p = FDM_TO_Z) {
+    const FdmPlan::Lists& L = *pl->sets[set].cur;
+    for (int k = mode == WAVE_Y ? 2 : 0, e = k + 2; k < e; k++) {
+        int rc = launch_wave(mode, k % 2 == 1, pl->d_wtasks.as<WaveTask>(), L.wave[k], L.n_wave[k], L.lds[k], s, skip,
+                             to_p);
+        if (rc) return rc;
+    }
+    return SE_OK;
+}
 
+// z = FDM(r) of the listed members: three wave kernels, or four dense passes
 // (to_p: into the CG's p, for a first or restarted direction; corr: in the
 // corrections' precision, for the residual of an update)
 int plan_fdm(FdmPlan* pl, int set, hipStream_t s, int skip = 0, int to_p = FDM_TO_Z, bool corr = false) {
+    for (int mode : {WAVE_X, WAVE_Y, WAVE_XB}) {
+        int rc = plan_wave(pl, set, mode, s, skip, to_p);
+        if (rc) return rc;
+    }
     for (int pass = 0; pass < 4; pass++) {
         int rc = plan_pass(pl, set, pass, s, skip, to_p, corr);
         if (rc) return rc;
@@ -1471,7 +1790,7 @@ int fdm_plan_solve(FdmPlan* pl, const double* const* d_f, double* const* d_x, co
     const int null = o.null_space ? 1 : 0;
     for (int i = 0; i < count; i++) {
         int rc = fdm_prepare(pl->ops[i], prec);
-        if (!rc && cprec != prec) rc = fdm_prepare(pl->ops[i], cprec);
+        if (!rc && cprec != prec && !fdm_wave(pl->ops[i], prec)) rc = fdm_prepare(pl->ops[i], cprec);
         if (rc) return rc;
     }
     // descriptors: built once per members / precision / null flag / tolerance;
@@ -1487,6 +1806,7 @@ int fdm_plan_solve(FdmPlan* pl, const double* const* d_f, double* const* d_x, co
                 if (pl->b_alias[i] && M.f != d_f[i]) {
                     M.b = const_cast<double*>(d_f[i]);  // read only: b is f
                     pl->h_tasks[4 * (size_t)i + 3].b = M.b;
+                    pl->h_wtasks[i].b = M.b;
                     bmoved = true;
                 }
                 M.f = d_f[i];
@@ -1500,9 +1820,12 @@ int fdm_plan_solve(FdmPlan* pl, const double* const* d_f, double* const* d_x, co
         if (changed && count > 0)
             SE_HIP(hipMemcpyAsync(pl->d_members.ptr, pl->h_members.data(), sizeof(FbMember) * count,
                                   hipMemcpyHostToDevice, s));
-        if (bmoved)
+        if (bmoved) {
             SE_HIP(hipMemcpyAsync(pl->d_tasks.ptr, pl->h_tasks.data(), sizeof(GemmTask) * 4 * count,
                                   hipMemcpyHostToDevice, s));
+            SE_HIP(hipMemcpyAsync(pl->d_wtasks.ptr, pl->h_wtasks.data(), sizeof(WaveTask) * count,
+                                  hipMemcpyHostToDevice, s));
+        }
         if (moved || bmoved) {  // the A x descriptors name the iterates and b
             int e = upload_apply_descriptors(pl, s);
             if (e) return e;
@@ -1518,6 +1841,11 @@ int fdm_plan_solve(FdmPlan* pl, const double* const* d_f, double* const* d_x, co
             int e = pl->d_tasks_c.alloc(sizeof(GemmTask) * 4 * std::max(count, 1));
             if (e) return e;
         }
+        {
+            int e = pl->d_wtasks.alloc(sizeof(WaveTask) * std::max(count, 1));
+            if (e) return e;
+        }
+        pl->h_wtasks.assign(count, WaveTask{});
         pl->any_svv = false;
         for (se_op* op : pl->ops) pl->any_svv = pl->any_svv || op->svv_mN != 0;
         pl->b_alias.assign(count, 0);
@@ -1550,11 +1878,23 @@ int fdm_plan_solve(FdmPlan* pl, const double* const* d_f, double* const* d_x, co
             M.nch = (std::max(M.n, 1) + FB_CH - 1) / FB_CH;
             M.fused = op->svv_mN == 0;
             M.nap = M.fused ? line_tiles(op->mesh->N, op->mesh->nEls[0], op->mesh->nEls[1]) : M.nch;
-            M.ntz = fdm_tiles(op);
+            M.wave = fdm_wave(op, prec);
+            M.ntz = M.wave ? wave_blocks(op, WAVE_X) : fdm_tiles(op);
+            M.ntr = M.wave ? wave_blocks(op, WAVE_Y) : M.ntz;
             M.null_space = null;
             M.sgn = (double)op->sign;
             M.rtol = o.rtol;
             M.st = pl->d_states.as<CgState>() + i;
+            if (M.wave) {
+                WaveTask w = wave_task(op, M.r, M.z, M.pz, null);
+                w.b = M.b;
+                w.p = M.p;
+                w.pv = M.pv;
+                w.st = M.st;
+                w.nch = M.nch;
+                pl->h_wtasks[i] = w;
+                continue;
+            }
             GemmTask t4[4];
             fdm_tasks(op, prec, M.r, M.z, M.pz, t4);
             SE_CHECK(fdm_tasks_valid(t4, prec), SE_ERR_STATE, "FDM: transform shapes break the kernels' assumptions");
@@ -1585,6 +1925,8 @@ int fdm_plan_solve(FdmPlan* pl, const double* const* d_f, double* const* d_x, co
                                   s));
             SE_HIP(hipMemcpyAsync(pl->d_tasks.ptr, tasks.data(), sizeof(GemmTask) * 4 * count, hipMemcpyHostToDevice, s));
             pl->h_tasks = tasks;
+            SE_HIP(hipMemcpyAsync(pl->d_wtasks.ptr, pl->h_wtasks.data(), sizeof(WaveTask) * count,
+                                  hipMemcpyHostToDevice, s));
             if (cprec != prec)
                 SE_HIP(hipMemcpyAsync(pl->d_tasks_c.ptr, tasks_c.data(), sizeof(GemmTask) * 4 * count,
                                       hipMemcpyHostToDevice, s));
@@ -1787,23 +2129,29 @@ int fdm_plan_probe(FdmPlan* pl, int reps, double* us_pass, double* flops_pass, d
     std::vector<char> all(count, 1);
     int rc = plan_lists(pl, FdmPlan::SET_OTHER, all, s);
     if (rc) return rc;
+    // the four 1-D transforms; a wave kernel that does two counts half for each
+    const bool wave = count > 0 && pl->h_members[0].wave;
     for (int pass = 0; pass < 4; pass++) {
+        const int mode = pass == 0 ? WAVE_X : (pass == 3 ? WAVE_XB : WAVE_Y);
+        auto once = [&]() {
+            return wave ? plan_wave(pl, FdmPlan::SET_OTHER, mode, s) : plan_pass(pl, FdmPlan::SET_OTHER, pass, s);
+        };
         double fl = 0.0;
         for (se_op* op : pl->ops) {
             const double nP0 = op->fdm->nP0, nP1 = op->fdm->nP1;
-            fl += 2.0 * nP0 * nP1 * ((pass == 0 || pass == 3) ? nP0 : nP1);
+            fl += wave ? wave_flops(op, mode == WAVE_Y ? 1 : 0) : 2.0 * nP0 * nP1 * ((pass == 0 || pass == 3) ? nP0 : nP1);
         }
         flops_pass[pass] = fl;
-        rc = plan_pass(pl, FdmPlan::SET_OTHER, pass, s);
+        rc = once();
         if (rc) return rc;
         SE_HIP(hipEventRecord(c->ev0, s));
-        for (int r = 0; r < reps && !rc; r++) rc = plan_pass(pl, FdmPlan::SET_OTHER, pass, s);
+        for (int r = 0; r < reps && !rc; r++) rc = once();
         SE_HIP(hipEventRecord(c->ev1, s));
         SE_HIP(hipEventSynchronize(c->ev1));
         if (rc) return rc;
         float ms = 0.f;
         (void)hipEventElapsedTime(&ms, c->ev0, c->ev1);
-        us_pass[pass] = 1e3 * ms / reps;
+        us_pass[pass] = 1e3 * ms / reps * (wave && mode == WAVE_Y ? 0.5 : 1.0);
     }
     double by = 0.0;
     for (se_op* op : pl->ops) by += 16.0 * op->mesh->n;
@@ -1826,7 +2174,6 @@ int fdm_plan_probe(FdmPlan* pl, int reps, double* us_pass, double* flops_pass, d
 int pcg_fdm(se_op* op, const double* d_f, double* d_x, const se_solve_opts& o, se_solve_info& info) {
     SE_CHECK(op->definite, SE_ERR_UNSUPPORTED, "operator diagonal changes sign: not a definite system");
     int rc = fdm_prepare(op, fdm_prec_of(o.precision));
-    if (!rc && fdm_cprec_of(o.precision) != fdm_prec_of(o.precision)) rc = fdm_prepare(op, fdm_cprec_of(o.precision));
     if (rc) return rc;
     if (!op->fdm->self) {
         rc = fdm_plan_create(op->mesh->ctx, 1, &op, &op->fdm->self);
@@ -1857,10 +2204,25 @@ extern "C" int se_helm_apply_fdm(se_op* op, int precision, const double* r, doub
     hipStream_t s = op->mesh->ctx->stream;
     SE_HIP(hipStreamSynchronize(s));
     if (n > 0) SE_HIP(hipMemcpy(op->r.ptr, r, sizeof(double) * n, hipMemcpyHostToDevice));
+    DevBuf d;
+    if (fdm_wave(op, prec)) {
+        const WaveTask w = wave_task(op, op->r.as<double>(), op->fdm->z.as<double>(), op->fdm->pz.as<double>(), 0);
+        rc = d.alloc(sizeof(w));
+        if (rc) return rc;
+        SE_HIP(hipMemcpy(d.ptr, &w, sizeof(w), hipMemcpyHostToDevice));
+        for (int mode : {WAVE_X, WAVE_Y, WAVE_XB}) {
+            const se_wave::Line& L = mode == WAVE_Y ? op->fdm->wy->L : op->fdm->wx->L;
+            rc = launch_wave(mode, wave_long(L.E), d.as<WaveTask>(), nullptr, wave_blocks(op, mode), wave_lds_of(op, mode), s, 0, FDM_TO_Z);
+            if (rc) return rc;
+        }
+        SE_HIP(hipGetLastError());
+        SE_HIP(hipStreamSynchronize(s));
+        if (n > 0) SE_HIP(hipMemcpy(z, op->fdm->z.ptr, sizeof(double) * n, hipMemcpyDeviceToHost));
+        return SE_OK;
+    }
     GemmTask t[4];
     fdm_tasks(op, prec, op->r.as<double>(), op->fdm->z.as<double>(), op->fdm->pz.as<double>(), t);
     SE_CHECK(fdm_tasks_valid(t, prec), SE_ERR_STATE, "se_helm_apply_fdm: transform shapes break the kernels' assumptions");
-    DevBuf d;
     rc = d.alloc(sizeof(t));
     if (rc) return rc;
     SE_HIP(hipMemcpy(d.ptr, t, sizeof(t), hipMemcpyHostToDevice));
