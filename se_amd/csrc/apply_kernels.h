@@ -59,6 +59,7 @@ __device__ __forceinline__ void reduce_partials(const double* __restrict__ parti
 #pragma unroll
     for (int k = 0; k < K; k++) {
         double s = 0.0;
+#pragma unroll 4
         for (int b = threadIdx.x; b < np; b += BS) s += partials[(size_t)k * np + b];
         s = wave_sum(s);
         if (lane == 0) s_red2[k][wid] = s;

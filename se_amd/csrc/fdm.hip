@@ -427,6 +427,25 @@ __device__ __forceinline__ void put_packed_c(const FbMember& M, int i, double v)
     put_packed_to(M, M.rpc, M.rcprec, i, v);
 }
 
+// A chunk is 16 unknowns a thread, taken eight at a time: all loads of the
+// eight before the first store (to the compiler the vectors may overlap, and
+// one by one an update's chain of loads and stores took 17 us at any size).
+constexpr int FB_U = 8;
+template <typename LOAD, typename STORE>
+__device__ __forceinline__ void fb_each(int i0, int i1, LOAD&& load, STORE&& store) {
+    for (int i = i0 + threadIdx.x; i < i1; i += FB_U * FB_NT) {
+        decltype(load(0)) v[FB_U];
+#pragma unroll
+        for (int u = 0; u < FB_U; u++) v[u] = load(min(i + u * FB_NT, i1 - 1));
+#pragma unroll
+        for (int u = 0; u < FB_U; u++)
+            if (i + u * FB_NT < i1) store(i + u * FB_NT, v[u]);
+    }
+}
+struct Fb4 {
+    double p, q, r, x;
+};
+
 __device__ __forceinline__ void chunk_range(const FbMember& M, int ch, int& i0, int& i1) {
     i0 = ch * FB_CH;
     i1 = min(M.n, i0 + FB_CH);
@@ -466,12 +485,17 @@ __global__ __launch_bounds__(FB_NT) void k_fb_start(const FbMember* __restrict__
         int i0, i1;
         chunk_range(M, it.y, i0, i1);
         double rr = 0.0;
-        for (int i = i0 + threadIdx.x; i < i1; i += FB_NT) {
-            const double bi = M.sgn * M.f[i] - mu;
-            if (M.b != M.f) M.b[i] = bi;  // (else b is f, and bi = f[i])
-            put_packed(M, i, bi);
-            rr += bi * bi;
-        }
+        const SE_GLOBAL double* f = gview(M.f);
+        SE_GLOBAL double* b = gview(M.b);
+        const bool keep = M.b != M.f, pack = !M.wave;
+        const double sgn = M.sgn;
+        fb_each(i0, i1, [&](int i) { return f[i]; },
+                [&](int i, double v) {
+                    const double bi = sgn * v - mu;
+                    if (keep) b[i] = bi;  // (else b is f, and bi = f[i])
+                    if (pack) put_packed(M, i, bi);
+                    rr += bi * bi;
+                });
         const double v[1] = {rr};
         block_store_partials_at<1, FB_NT>(v, M.pv, it.y, M.nch);
     }
@@ -569,7 +593,10 @@ __global__ __launch_bounds__(FB_NT) void k_fb_dir(const FbMember* __restrict__ M
             continue;
         }
         if (mode == FB_NORMAL) {
-            for (int i = i0 + threadIdx.x; i < i1; i += FB_NT) M.p[i] = (M.z[i] - mu) + beta * M.p[i];
+            const SE_GLOBAL double* z = gview(M.z);
+            SE_GLOBAL double* p = gview(M.p);
+            fb_each(i0, i1, [&](int i) { return Fb4{p[i], 0.0, 0.0, z[i]}; },
+                    [&](int i, const Fb4& v) { p[i] = (v.x - mu) + beta * v.p; });
         } else if (mu != 0.0) {  // the transforms wrote z into p
             for (int i = i0 + threadIdx.x; i < i1; i += FB_NT) M.p[i] -= mu;
         }
@@ -629,13 +656,17 @@ __global__ __launch_bounds__(FB_NT) void k_fb_update(const FbMember* __restrict_
             st->rho_prev = rho;
         }
         double rr = 0.0;
-        for (int i = i0 + threadIdx.x; i < i1; i += FB_NT) {
-            M.x[i] = first ? alpha * M.p[i] : M.x[i] + alpha * M.p[i];
-            const double ri = (first ? M.b[i] : M.r[i]) - alpha * M.q[i];
-            M.r[i] = ri;
-            put_packed_c(M, i, ri);
-            rr += ri * ri;
-        }
+        const SE_GLOBAL double *p = gview(M.p), *q = gview(M.q), *ro = gview(first ? M.b : M.r);
+        SE_GLOBAL double *x = gview(M.x), *r = gview(M.r);
+        const bool pack = !M.wave;
+        fb_each(i0, i1, [&](int i) { return Fb4{p[i], q[i], ro[i], first ? 0.0 : x[i]}; },
+                [&](int i, const Fb4& v) {
+                    x[i] = first ? alpha * v.p : v.x + alpha * v.p;
+                    const double ri = v.r - alpha * v.q;
+                    r[i] = ri;
+                    if (pack) put_packed_c(M, i, ri);
+                    rr += ri * ri;
+                });
         const double v[1] = {rr};
         block_store_partials_at<1, FB_NT>(v, M.pv, it.y, M.nch);
     }

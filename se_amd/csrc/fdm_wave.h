@@ -87,14 +87,21 @@ __host__ __device__ inline size_t wave_lds(int N, int E, int E16, int LD) {
 // wave, all K steps.  Operands of zero stand where a block has fewer rows than
 // its tiles; the LDS rows they meet hold finite values (other blocks' or
 // cleared rows).
+constexpr int kWaveUN = 2;  // K steps a group of operands covers
+template <int NA>
+struct WaveTiles {
+    WaveTile t[NA];
+    double a[kWaveUN][NA];  // the first group of operands
+};
 template <int NQ, int NA, bool FWD>
-__device__ __forceinline__ void wave_product(const WaveDim& d, const double* U, const WaveTile (&t)[NA],
+__device__ __forceinline__ void wave_product(const WaveDim& d, const double* U, const WaveTiles<NA>& w,
                                              wave_f64x4 (&acc)[NA], int l) {
+    const WaveTile(&t)[NA] = w.t;
     const int KS = FWD ? d.kf : d.kb;
     const SE_GLOBAL double* A = gview(FWD ? d.fwd : d.bwd) + l;
     const double* B = U + (l & 15);
     // the wave matrix's operands are loaded UN steps ahead
-    constexpr int UN = 2;
+    constexpr int UN = kWaveUN;
     double a[2][UN][NQ];
     auto load_a = [&](int h, int ks) {
 #pragma unroll
@@ -120,7 +127,10 @@ __device__ __forceinline__ void wave_product(const WaveDim& d, const double* U, 
             for (int q = 0; q < NQ; q++)
                 acc[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[h][u][q], b[u][q], acc[q], 0, 0, 0);
     };
-    load_a(0, 0);
+#pragma unroll
+    for (int u = 0; u < UN; u++)
+#pragma unroll
+        for (int q = 0; q < NQ; q++) a[0][u][q] = w.a[u][q];
     for (int ks = 0; ks < KS; ks += 2 * UN) {  // (KS is a multiple of UN)
         if (ks + UN < KS) load_a(1, ks + UN);
         multiply(0, ks);
@@ -130,33 +140,45 @@ __device__ __forceinline__ void wave_product(const WaveDim& d, const double* U, 
     }
 }
 
-// the eight waves share the tiles; every wave is past its reads of U before
-// the results go over it
-template <bool FWD, bool LONG>
-__device__ __forceinline__ void wave_matrix(double* U, const WaveDim& d) {
-    constexpr int NA = LONG ? 7 : 4;
+// This wave's tiles of a product and the first of their operands, loaded well
+// before the product (behind the lines' loads, the N x N matrices).
+template <bool FWD, int NA>
+__device__ __forceinline__ void wave_ahead(const WaveDim& d, WaveTiles<NA>& w) {
     const int l = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int nt = FWD ? d.nf : d.nb;
     typedef const __attribute__((address_space(4))) WaveTile ctile;  // (uniform: scalar loads)
     ctile* tab = (ctile*)(FWD ? d.tf : d.tb);
-    WaveTile t[NA];
-    wave_f64x4 acc[NA];
+    const SE_GLOBAL double* A = gview(FWD ? d.fwd : d.bwd) + l;
 #pragma unroll
     for (int q = 0; q < NA; q++) {
         ctile& c = tab[min(wv + 8 * q, nt - 1)];
-        t[q] = WaveTile{c.of, c.col, c.w, c.row, c.at, c.step, c.b0, c.cnt};
-        acc[q] = wave_f64x4{0.0, 0.0, 0.0, 0.0};
+        w.t[q] = WaveTile{c.of, c.col, c.w, c.row, c.at, c.step, c.b0, c.cnt};
+#pragma unroll
+        for (int u = 0; u < kWaveUN; u++) w.a[u][q] = A[w.t[q].of + u * 64];
     }
+}
+
+// the eight waves share the tiles; every wave is past its reads of U before
+// the results go over it
+template <bool FWD, int NA>
+__device__ __forceinline__ void wave_matrix(double* U, const WaveDim& d, const WaveTiles<NA>& w) {
+    constexpr bool LONG = NA > 4;
+    const int l = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int nt = FWD ? d.nf : d.nb;
+    const WaveTile(&t)[NA] = w.t;
+    wave_f64x4 acc[NA];
+#pragma unroll
+    for (int q = 0; q < NA; q++) acc[q] = wave_f64x4{0.0, 0.0, 0.0, 0.0};
     const int mine = (nt - wv + 7) >> 3;
     if (LONG) {
-        wave_product<NA, NA, FWD>(d, U, t, acc, l);
+        wave_product<NA, NA, FWD>(d, U, w, acc, l);
     } else {
         switch (mine) {
             case 0: break;
-            case 1: wave_product<1, NA, FWD>(d, U, t, acc, l); break;
-            case 2: wave_product<2, NA, FWD>(d, U, t, acc, l); break;
-            case 3: wave_product<3, NA, FWD>(d, U, t, acc, l); break;
-            default: wave_product<NA, NA, FWD>(d, U, t, acc, l); break;
+            case 1: wave_product<1, NA, FWD>(d, U, w, acc, l); break;
+            case 2: wave_product<2, NA, FWD>(d, U, w, acc, l); break;
+            case 3: wave_product<3, NA, FWD>(d, U, w, acc, l); break;
+            default: wave_product<NA, NA, FWD>(d, U, w, acc, l); break;
         }
     }
     __syncthreads();
@@ -407,6 +429,9 @@ __global__ __launch_bounds__(kWaveT, LONG ? 2 : 4) void k_fdm_wave(const WaveTas
         auto in_t1 = [&](int J) { return (((size_t)(J >> lgx) * nMx + line) << lgx) + (J & (Rx - 1)); };
         double* U = wave_u + kWavePad * d.LD;
         double* Phi = U + d.E16 * d.LD + 16;
+        WaveTiles<LONG ? 7 : 4> tiles;
+        if (MODE == WAVE_XB) wave_ahead<false>(d, tiles);
+        else wave_ahead<true>(d, tiles);
         __syncthreads();  // the previous item is done with U
         if (MODE == WAVE_X) {
             const SE_GLOBAL double* src = gview(to_p == 2 ? t.b : t.r) + (size_t)line * d.n;
@@ -424,7 +449,8 @@ __global__ __launch_bounds__(kWaveT, LONG ? 2 : 4) void k_fdm_wave(const WaveTas
             for (int k = threadIdx.x; k < (t.N * t.N * d.E16) >> 1; k += kWaveT) ((wave_d2*)Phi)[k] = f[k];
         }
         __syncthreads();
-        if (MODE != WAVE_XB) wave_matrix<true, LONG>(U, d);
+        if (MODE != WAVE_XB) wave_matrix<true>(U, d, tiles);
+        if (MODE == WAVE_Y) wave_ahead<false>(d, tiles);
         const double rz = wave_modes_n<MODE, LONG>(t, d, U, Phi, it.y);
         if (MODE == WAVE_Y) {
             const double v[1] = {rz};
@@ -435,7 +461,7 @@ __global__ __launch_bounds__(kWaveT, LONG ? 2 : 4) void k_fdm_wave(const WaveTas
             wave_block<true>(t, d, U, it.y);
             continue;
         }
-        wave_matrix<false, LONG>(U, d);
+        wave_matrix<false>(U, d, tiles);
         if (MODE == WAVE_Y) {
             SE_GLOBAL double* T = gview(t.t1);
             wave_unfold<false>(t, d, U, ok, [&](int J, double v) { T[in_t1(J)] = v; });
