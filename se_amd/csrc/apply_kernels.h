@@ -85,6 +85,7 @@ struct ApplyMember {
     const double* b = nullptr;   // AP_TRUE: the right-hand side
     const CgState* gate = nullptr;  // gated launches: only while this CG awaits its true residual
     int np = 0;
+    int N = 0;                   // the order (k_apply_lines_any)
 };
 
 }  // namespace se

@@ -164,8 +164,20 @@ __device__ __forceinline__ void line_outputs(const OpParams& P, const double* s_
     }
 }
 
+// LDS of a tile
+template <int N>
+struct LineLds {
+    static constexpr int TX = LineShape<N>::TX, TY = LineShape<N>::TY, N1 = N + 1, NP = N1 * N1;
+    static constexpr int BWU = (TX + 1) * N + 1, BH = (TY + 1) * N + 1;
+    double u[BH * (BWU | 1)];           // the node block, odd row pitch
+    double o[(TX + 1) * (TY + 1) * NP];  // FP32 exchange, then the element outputs
+    double cf[(TX + 1) * 4 * N1], rf[(TY + 1) * 4 * N1];
+    float cq[(TX + 1) * 2 * NP], rq[(TY + 1) * 2 * NP];
+    int I[BWU], J[BH];  // unknown column / row of each block column / row (-1: none)
+};
+
 template <int N, int MODE>
-__device__ __forceinline__ void apply_lines_tile(const OpParams& P, int tile,
+__device__ __forceinline__ void apply_lines_tile(LineLds<N>& lds, int tid, const OpParams& P, int tile,
                                                  const double* __restrict__ in, double* __restrict__ out,
                                                  double* __restrict__ partials, int np,
                                                  const double* __restrict__ b = nullptr) {
@@ -178,15 +190,12 @@ __device__ __forceinline__ void apply_lines_tile(const OpParams& P, int tile,
     constexpr int F = 4 * N1;                   // line factors A0 A1 A2 AM (Y0 Y1 Y2w MY)
     constexpr int QS = 2 * NP;                  // FP32 cross tables: Q, Q transposed
 
-    __shared__ double s_u[BH * BW];
-    __shared__ double s_o[NE * NP];              // FP32 exchange, then the element outputs
-    __shared__ double s_cf[(TX + 1) * F], s_rf[(TY + 1) * F];
-    __shared__ float s_cq[(TX + 1) * QS], s_rq[(TY + 1) * QS];
-    __shared__ int s_I[BWU], s_J[BH];            // unknown column / row of each block column / row (-1: none)
+    double *s_u = lds.u, *s_o = lds.o, *s_cf = lds.cf, *s_rf = lds.rf;
+    float *s_cq = lds.cq, *s_rq = lds.rq;
+    int *s_I = lds.I, *s_J = lds.J;
     float* s_xf = (float*)s_o;                   // u_xi  [e][qx][qy]
     float* s_ef = s_xf + NE * NP;                // u_eta [e][qy][qx]
 
-    const int tid = threadIdx.x;
     const int tilesX = (P.nEls0 + TX - 1) / TX;
     const int ex0 = (tile % tilesX) * TX, ey0 = (tile / tilesX) * TY;
     const int txo = min(TX, P.nEls0 - ex0), tyo = min(TY, P.nEls1 - ey0);
@@ -313,16 +322,26 @@ template <int N, bool DOT>
 __global__ __launch_bounds__(256) void k_apply_lines(OpParams P, const double* __restrict__ in,
                                                       double* __restrict__ out, double* __restrict__ partials,
                                                       const CgState* __restrict__ st) {
+    __shared__ LineLds<N> lds;
     if (DOT && cg_stopped(st)) return;
     // workgroup b runs on XCD b mod 8: give each XCD a contiguous run of
     // tiles, so that neighbouring tiles' shared halo lines meet in one L2
     const int T = gridDim.x, b = blockIdx.x, q = T / 8, r = T % 8, x = b % 8;
     const int tile = x * q + min(x, r) + b / 8;
-    apply_lines_tile<N, DOT ? AP_DOT : AP_PLAIN>(P, tile, in, out, partials, T);
+    apply_lines_tile<N, DOT ? AP_DOT : AP_PLAIN>(lds, threadIdx.x, P, tile, in, out, partials, T);
 }
 
-// Batched: work items (member, tile) over members of one order; MODE's
-// partials go to the member's `part` (line_tiles of its mesh entries).
+// The thread, hidden from the compiler: each tile of a work list derives its
+// indices anew (kept over the list's loop, of every order in
+// k_apply_lines_any, they spilled up to 167 registers).
+__device__ __forceinline__ int opaque_tid() {
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    return tid;
+}
+
+// Batched: work items (member, tile); MODE's partials go to the member's
+// `part` (line_tiles of its mesh entries).
 // gated: a member whose `gate` CG is not awaiting its true-residual check
 // (the direction kernel before this launch marks it) has nothing to do.
 // Four workgroups per CU (at most 128 VGPRs; at N = 8 a few values spill to
@@ -330,13 +349,46 @@ __global__ __launch_bounds__(256) void k_apply_lines(OpParams P, const double* _
 template <int N, int MODE>
 __global__ __launch_bounds__(256, 4) void k_apply_lines_batch(const ApplyMember* __restrict__ members,
                                                             const int2* __restrict__ work, int nwork, int gated) {
+    __shared__ LineLds<N> lds;
     for (int w = blockIdx.x; w < nwork; w += gridDim.x) {
         const int2 it = work[w];
         if (it.x < 0) continue;  // a padding item of an XCD-ordered list
         const ApplyMember& a = members[it.x];
         if (gated && a.gate && a.gate->status != CG_PENDING) continue;
         __syncthreads();  // the previous item's LDS reads are done
-        apply_lines_tile<N, MODE>(a.P, it.y, a.in, a.out, a.part, a.np, a.b);
+        apply_lines_tile<N, MODE>(lds, opaque_tid(), a.P, it.y, a.in, a.out, a.part, a.np, a.b);
+    }
+}
+
+// The same over members of any orders at once: the orders' tiles run side by
+// side, where a launch per order left most of the chip idle and cost 8-18 us
+// each at small sizes (24 channel states of six orders: 78 -> 19 us; the
+// 512-member ensemble, three orders of many tiles each, is unchanged).  One
+// LDS pool, the largest order's: N = 8 holds four workgroups a CU either way.
+template <int MODE>
+__global__ __launch_bounds__(256, 4) void k_apply_lines_any(const ApplyMember* __restrict__ members,
+                                                          const int2* __restrict__ work, int nwork, int gated) {
+    __shared__ union {
+        LineLds<2> l2;
+        LineLds<3> l3;
+        LineLds<4> l4;
+        LineLds<5> l5;
+        LineLds<6> l6;
+        LineLds<7> l7;
+        LineLds<8> l8;
+    } lds;
+    for (int w = blockIdx.x; w < nwork; w += gridDim.x) {
+        const int2 it = work[w];
+        if (it.x < 0) continue;  // a padding item of an XCD-ordered list
+        const ApplyMember& a = members[it.x];
+        if (gated && a.gate && a.gate->status != CG_PENDING) continue;
+        __syncthreads();  // the previous item's LDS reads are done
+        switch (a.N) {
+#define SE_CASE(NN)                                                                         \
+    case NN: apply_lines_tile<NN, MODE>(lds.l##NN, opaque_tid(), a.P, it.y, a.in, a.out, a.part, a.np, a.b); break;
+            SE_CASE(2) SE_CASE(3) SE_CASE(4) SE_CASE(5) SE_CASE(6) SE_CASE(7) SE_CASE(8)
+#undef SE_CASE
+        }
     }
 }
 

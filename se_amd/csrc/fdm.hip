@@ -1373,16 +1373,10 @@ struct FdmPlan {
     DevBuf d_wtasks;            // WaveTask[count]; of a wave-form member the GemmTasks are unused
     std::vector<WaveTask> h_wtasks;
     std::vector<FbMember> h_members;
-    // FP64 apply descriptors per order (p -> q and x -> q)
-    struct Order {
-        int N;
-        std::vector<int> members;
-        DevBuf d_ap, d_ax;  // ApplyMember[]
-    };
-    std::vector<Order> orders;   // one per order 2..8 (members may be empty)
+    DevBuf d_ap, d_ax;  // FP64 apply descriptors ApplyMember[count] (p -> q and x -> q)
     // Work lists of one member subset: (member, chunk) items of the vector
-    // kernels, (member, tile) items of the transforms, per order the apply's
-    // (local member, tile) items, and the member list, packed in one device
+    // kernels, (member, tile) items of the transforms and of the apply,
+    // and the member list, packed in one device
     // buffer.  Two independent sets -- the running members' iteration with
     // its true-residual checks, and restarts and the end of a solve -- each keep the
     // lists of the last kListCache subsets they were asked for (successive
@@ -1396,9 +1390,9 @@ struct FdmPlan {
     struct Lists {
         std::vector<char> on;  // the member flags these lists were built for
         DevBuf d;
-        const int2 *vwork = nullptr, *gwork = nullptr, *wave[4] = {}, *apply[7] = {};
+        const int2 *vwork = nullptr, *gwork = nullptr, *wave[4] = {}, *apply = nullptr;
         const int* list = nullptr;
-        int n_vwork = 0, n_gwork = 0, n_wave[4] = {}, n_apply[7] = {}, n_list = 0;
+        int n_vwork = 0, n_gwork = 0, n_wave[4] = {}, n_apply = 0, n_list = 0;
         size_t lds[4] = {};  // wave lists: x lines, long x lines, y, long y; the largest line block of each
         unsigned long long used = 0;
     };
@@ -1446,27 +1440,11 @@ struct FdmPlan {
 
 namespace {
 
-template <int MODE>
-int launch_apply_batch_m(int N, const ApplyMember* A, const int2* work, int nw, int grid, hipStream_t s, int gated) {
-    switch (N) {
-#define SE_CASE(NN)                                                                                        \
-    case NN:                                                                                               \
-        hipLaunchKernelGGL((k_apply_lines_batch<NN, MODE>), dim3(grid), dim3(256), 0, s, A, work, nw, gated); \
-        break;
-        SE_CASE(2) SE_CASE(3) SE_CASE(4) SE_CASE(5) SE_CASE(6) SE_CASE(7) SE_CASE(8)
-#undef SE_CASE
-        default: return fail(SE_ERR_UNSUPPORTED, "FDM solve built for orders 2..8");
-    }
-    return SE_OK;
-}
-
 // (grid <= nw workgroups; a multiple of 8 below nw, so that a workgroup's
 // items keep its XCD's place in the XCD-ordered list)
-int launch_apply_batch(int N, int mode, const ApplyMember* A, const int2* work, int nw, int grid, hipStream_t s,
-                       int gated) {
-    if (mode == AP_DOT) return launch_apply_batch_m<AP_DOT>(N, A, work, nw, grid, s, gated);
-    if (mode == AP_TRUE) return launch_apply_batch_m<AP_TRUE>(N, A, work, nw, grid, s, gated);
-    return launch_apply_batch_m<AP_PLAIN>(N, A, work, nw, grid, s, gated);
+void launch_apply_any(int mode, const ApplyMember* A, const int2* work, int nw, int grid, hipStream_t s, int gated) {
+    auto k = mode == AP_DOT ? k_apply_lines_any<AP_DOT> : k_apply_lines_any<AP_TRUE>;
+    hipLaunchKernelGGL(k, dim3(grid), dim3(256), 0, s, A, work, nw, gated);
 }
 
 // Work lists XCD by XCD.  The dispatcher hands workgroup b to XCD b mod 8
@@ -1530,18 +1508,14 @@ void xcd_interleave(const std::vector<int>& ids, const std::vector<int>& tiles, 
 int plan_apply(FdmPlan* pl, int set, bool from_x, hipStream_t s, bool gated = false) {
     const FdmPlan::Lists& L = *pl->sets[set].cur;
     const int mode = from_x ? AP_TRUE : AP_DOT;
-    for (int k = 0; k < (int)pl->orders.size(); k++) {
-        const FdmPlan::Order& o = pl->orders[k];
-        const int nw = L.n_apply[k];
-        if (o.members.empty() || nw == 0) continue;
-        const ApplyMember* A = from_x ? o.d_ax.as<ApplyMember>() : o.d_ap.as<ApplyMember>();
+    const int nw = L.n_apply;
+    if (nw > 0) {
         // a gated check runs for few members, if any: one workgroup per resident
         // slot (four per CU) walks the list, instead of one per tile whose
         // dispatch alone costs ~20 us at the ensemble's 14 k tiles
         const int slots = std::max(8, 4 * pl->ctx->cu_count / 8 * 8);
-        const int grid = gated ? std::min(nw, slots) : nw;
-        int rc = launch_apply_batch(o.N, mode, A, L.apply[k], nw, grid, s, gated ? 1 : 0);
-        if (rc) return rc;
+        launch_apply_any(mode, (from_x ? pl->d_ax : pl->d_ap).as<ApplyMember>(), L.apply, nw,
+                         gated ? std::min(nw, slots) : nw, s, gated ? 1 : 0);
     }
     // members with an SVV term: add it to the batched apply's result
     for (int i = 0; i < (int)pl->ops.size(); i++) {
@@ -1602,7 +1576,7 @@ int plan_lists(FdmPlan* pl, int set, const std::vector<char>& on, hipStream_t s)
             S.cur = e.get();
             return SE_OK;
         }
-    std::vector<int2> vwork, gwork, wave[4], apply[7];
+    std::vector<int2> vwork, gwork, wave[4], apply;
     std::vector<int> list;
     for (int i = 0; i < (int)pl->ops.size(); i++) {
         if (!on[i]) continue;
@@ -1612,26 +1586,25 @@ int plan_lists(FdmPlan* pl, int set, const std::vector<char>& on, hipStream_t s)
     xcd_order(pl, on, gwork);
     size_t lds[4];
     for (int k = 0; k < 4; k++) lds[k] = wave_order(pl, on, k, wave[k]);
-    for (int k = 0; k < (int)pl->orders.size(); k++) {
-        const FdmPlan::Order& o = pl->orders[k];
+    {
         std::vector<int> ids, tiles;
         std::vector<double> cost;
         std::vector<const void*> cls;
-        for (int j = 0; j < (int)o.members.size(); j++) {
-            const int i = o.members[j];
+        for (int i = 0; i < (int)pl->ops.size(); i++) {
             if (!on[i]) continue;
             const se_mesh* m = pl->ops[i]->mesh;
-            ids.push_back(j);
+            ids.push_back(i);
             tiles.push_back(line_tiles(m->N, m->nEls[0], m->nEls[1]));
-            cost.push_back((double)tiles.back());
+            // a tile costs its line threads' N + 1 products of N + 1
+            cost.push_back((double)tiles.back() * (m->N + 1) * (m->N + 1));
             cls.push_back(nullptr);
         }
-        xcd_interleave(ids, tiles, cost, cls, apply[k]);
+        xcd_interleave(ids, tiles, cost, cls, apply);
     }
     // packed: vector items, transform items, per-order apply items (int2), member list (int)
     size_t n2 = vwork.size() + gwork.size();
     for (const auto& w : wave) n2 += w.size();
-    for (const auto& a : apply) n2 += a.size();
+    n2 += apply.size();
     const size_t bytes = sizeof(int2) * n2 + sizeof(int) * list.size();
     if (bytes > S.hcap) {
         if (S.h) {
@@ -1669,10 +1642,8 @@ int plan_lists(FdmPlan* pl, int set, const std::vector<char>& on, hipStream_t s)
         L->n_wave[k] = (int)wave[k].size();
         L->lds[k] = lds[k];
     }
-    for (int k = 0; k < 7; k++) {
-        L->apply[k] = reinterpret_cast<const int2*>(put(apply[k].data(), sizeof(int2) * apply[k].size()));
-        L->n_apply[k] = (int)apply[k].size();
-    }
+    L->apply = reinterpret_cast<const int2*>(put(apply.data(), sizeof(int2) * apply.size()));
+    L->n_apply = (int)apply.size();
     L->list = reinterpret_cast<const int*>(put(list.data(), sizeof(int) * list.size()));
     L->n_vwork = (int)vwork.size();
     L->n_gwork = (int)gwork.size();
@@ -1731,16 +1702,8 @@ int plan_fdm(FdmPlan* pl, int set, hipStream_t s, int skip = 0, int to_p = FDM_T
 int fdm_plan_set_members(FdmPlan* pl, int count, se_op* const* ops) {
     SE_HIP(hipStreamSynchronize(pl->ctx->stream));  // nothing of the previous set is in flight
     pl->ops.assign(ops, ops + count);
-    if (pl->orders.empty()) {
-        pl->orders.resize(7);
-        for (int k = 0; k < 7; k++) pl->orders[k].N = k + 2;
-    }
-    for (auto& o : pl->orders) o.members.clear();
-    for (int i = 0; i < count; i++) {
-        const int N = ops[i]->mesh->N;
-        SE_CHECK(N >= 2 && N <= 8, SE_ERR_UNSUPPORTED, "FDM solve built for orders 2..8");
-        pl->orders[N - 2].members.push_back(i);
-    }
+    for (int i = 0; i < count; i++)
+        SE_CHECK(ops[i]->mesh->N >= 2 && ops[i]->mesh->N <= 8, SE_ERR_UNSUPPORTED, "FDM solve built for orders 2..8");
     if (count > pl->h_cap) {
         if (pl->h_states) (void)hipHostFree(pl->h_states);
         pl->h_states = nullptr;
@@ -1769,40 +1732,39 @@ int fdm_plan_create(se_ctx* c, int count, se_op* const* ops, FdmPlan** out) {
 
 void fdm_plan_destroy(FdmPlan* pl) { delete pl; }
 
-// the FP64 apply descriptors of every order group: A p (+ p.q partials) and
+// the FP64 apply descriptors: A p (+ p.q partials) and
 // A x (or, fused, the true residual), with each member's current iterate
 int upload_apply_descriptors(FdmPlan* pl, hipStream_t s) {
-    for (auto& od : pl->orders) {
-        if (od.members.empty()) continue;
-        std::vector<ApplyMember> ap, ax;
-        for (int i : od.members) {
-            se_op* op = pl->ops[i];
-            const FbMember& M = pl->h_members[i];
-            ApplyMember A;
-            A.P = op_params(op, (double)op->sign);
-            A.in = op->p.as<double>();
-            A.out = op->q.as<double>();
-            if (M.fused) {  // + partials of p.q
-                A.part = M.pa;
-                A.np = M.nap;
-            }
-            ap.push_back(A);
-            A.in = M.x;
-            A.gate = M.st;
-            if (M.fused) {  // r = b - A x, partials of sum t, sum t^2
-                A.out = op->r.as<double>();
-                A.b = M.b;
-                A.part = M.pt;
-            }
-            ax.push_back(A);
+    std::vector<ApplyMember> ap, ax;
+    for (size_t i = 0; i < pl->ops.size(); i++) {
+        se_op* op = pl->ops[i];
+        const FbMember& M = pl->h_members[i];
+        ApplyMember A;
+        A.P = op_params(op, (double)op->sign);
+        A.N = op->mesh->N;
+        A.in = op->p.as<double>();
+        A.out = op->q.as<double>();
+        if (M.fused) {  // + partials of p.q
+            A.part = M.pa;
+            A.np = M.nap;
         }
-        int rc = od.d_ap.alloc(sizeof(ApplyMember) * ap.size());
-        if (!rc) rc = od.d_ax.alloc(sizeof(ApplyMember) * ax.size());
-        if (rc) return rc;
-        SE_HIP(hipMemcpyAsync(od.d_ap.ptr, ap.data(), sizeof(ApplyMember) * ap.size(), hipMemcpyHostToDevice, s));
-        SE_HIP(hipMemcpyAsync(od.d_ax.ptr, ax.data(), sizeof(ApplyMember) * ax.size(), hipMemcpyHostToDevice, s));
-        SE_HIP(hipStreamSynchronize(s));  // the host vectors go out of scope
+        ap.push_back(A);
+        A.in = M.x;
+        A.gate = M.st;
+        if (M.fused) {  // r = b - A x, partials of sum t, sum t^2
+            A.out = op->r.as<double>();
+            A.b = M.b;
+            A.part = M.pt;
+        }
+        ax.push_back(A);
     }
+    if (ap.empty()) return SE_OK;
+    int rc = pl->d_ap.alloc(sizeof(ApplyMember) * ap.size());
+    if (!rc) rc = pl->d_ax.alloc(sizeof(ApplyMember) * ax.size());
+    if (rc) return rc;
+    SE_HIP(hipMemcpyAsync(pl->d_ap.ptr, ap.data(), sizeof(ApplyMember) * ap.size(), hipMemcpyHostToDevice, s));
+    SE_HIP(hipMemcpyAsync(pl->d_ax.ptr, ax.data(), sizeof(ApplyMember) * ax.size(), hipMemcpyHostToDevice, s));
+    SE_HIP(hipStreamSynchronize(s));  // the host vectors go out of scope
     return SE_OK;
 }
 
