@@ -203,6 +203,39 @@ SE_POW_FN double pow_int_at(const PowBase& b, int k) {
     return exp_hi_lo(ehi, elo, sign_bias);
 }
 
+// pow(x, k) where no special case can arise: 2^-60 <= |x| <= 1 and k <= 11, so
+// that log|x| is 0 or at least 2^-54 in size and k log|x| stays above -512.
+// The same operations as pow_int_at without its tests; pow(x, 1) is x (the
+// algorithm's error before its last rounding is far below half a unit).
+SE_POW_FN bool pow_plain(double x) { return fabs(x) >= 0x1p-60 && fabs(x) <= 1.0; }
+
+SE_POW_FN double pow_plain_at(double x, double hi, double lo, int k) {
+#pragma clang fp contract(off)
+    if (k == 0) return 1.0;
+    if (k == 1) return x;
+    const double InvLn2N = 0x1.71547652b82fep0 * 128, Shift = 0x1.8p52, NegLn2hiN = -0x1.62e42fefa0000p-8,
+                 NegLn2loN = -0x1.cf79abc9e3b3ap-47;
+    const double C2 = 0x1.ffffffffffdbdp-2, C3 = 0x1.555555555543cp-3, C4 = 0x1.55555cf172b91p-5,
+                 C5 = 0x1.1111167a4d017p-7;
+    const double y = (double)k;
+    const double ehi = y * hi;
+    const double elo = fma(y, lo, fma(y, hi, -ehi));
+    double kd = fma(InvLn2N, ehi, Shift);
+    const uint64_t ki = bits(kd);
+    kd -= Shift;
+    double r = fma(kd, NegLn2loN, fma(kd, NegLn2hiN, ehi));
+    r += elo;
+    const uint64_t idx = 2 * (ki % 128);
+    // an odd power carries x's sign
+    const uint64_t top = (ki << 45) + ((k & 1) ? bits(x) & 0x8000000000000000ULL : 0);
+    const double tail = from_bits(kPowExpTab[idx]);
+    const uint64_t sbits = kPowExpTab[idx + 1] + top;
+    const double r2 = r * r;
+    const double tmp = fma(r2 * r2, fma(r, C5, C4), fma(r2, fma(r, C3, C2), tail + r));
+    const double scale = from_bits(sbits);
+    return fma(scale, tmp, scale);
+}
+
 // pow(x, k) for an integer 0 <= k < 2^53
 SE_POW_FN double pow_int(double x, int k) {
     if (k == 0) return 1.0;

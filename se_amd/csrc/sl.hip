@@ -1,7 +1,7 @@
 // sl.hip -- semi-Lagrangian advection (departure-point search + GLL
 // interpolation), velocity from the stream function, CFL time step.
 //
-// One thread per field node.  The coordinate arithmetic that decides the
+// Two lanes per field node, one for each dimension.  The coordinate arithmetic that decides the
 // departure element (RK2 midpoint, wrap/clamp, GetEl's modf and its 1e-12
 // edge rule, the local-coordinate map) follows the reference's operation order
 // with FP contraction disabled.  P_N(x_j) is tabulated on the host with the
@@ -41,42 +41,68 @@ struct SLGeom {
 
 #define SE_NUMAPPROX(var, val) ((var) >= (val)-1.0e-12 && (var) <= (val) + 1.0e-12)
 
-// Mesh::GetEl, src/base/Mesh.cpp:106-137
-__device__ __forceinline__ int get_el(const SLGeom& g, double cx, double cy) {
+// One dimension of the mesh.  The departure-point kernels give every point a
+// pair of neighbouring lanes, the even one for x and the odd one for y: all of
+// a point's arithmetic but the sums over an element's nodes is separable, and
+// of those each lane sums its own component of a velocity.  With one lane per
+// node a mesh of 37 k nodes was one wave per SIMD walking a serial chain (powers,
+// divisions, sums), and at 332 k nodes 167 registers were wanted.
+struct Line {
+    int dim, nEls, per, n0;  // n0: nodes from one element to the next, N or N nv0
+    double min, max, dx, sc;  // sc = 2 / dx
+};
+
+template <int NN>
+__device__ __forceinline__ Line line_of(const SLGeom& g, int dim) {
 #pragma clang fp contract(off)
-    int t0, t1;
+    Line l;
+    l.dim = dim;
+    l.nEls = dim ? g.nEls1 : g.nEls0;
+    l.per = dim ? g.per1 : g.per0;
+    l.n0 = (NN ? NN : g.N) * (dim ? g.nv0 : 1);
+    l.min = dim ? g.min1 : g.min0;
+    l.max = dim ? g.max1 : g.max0;
+    l.dx = dim ? g.dx1 : g.dx0;
+    l.sc = 2.0 / l.dx;
+    return l;
+}
+
+// quad_perm of the doubles of a lane pair
+template <int CTRL>
+__device__ __forceinline__ double quad(double v) {
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+constexpr int kEven = 0xA0, kOdd = 0xF5, kSwap = 0xB1;  // [0,0,2,2], [1,1,3,3], [1,0,3,2]
+
+// Mesh::GetEl, src/base/Mesh.cpp:106-137, in one dimension
+__device__ __forceinline__ int get_el(const Line& l, double c) {
+#pragma clang fp contract(off)
+    int t;
     double integer, frac;
-    if (SE_NUMAPPROX(cx - g.max0, 0.0)) {
-        t0 = g.nEls0 - 1;
+    if (SE_NUMAPPROX(c - l.max, 0.0)) {
+        t = l.nEls - 1;
     } else {
-        double out = (cx - g.min0) / g.dx0;
+        double out = (c - l.min) / l.dx;
         frac = modf(out, &integer);
-        t0 = (int)integer;
-        if (t0 > 0 && SE_NUMAPPROX(frac, 0.0)) t0--;
-    }
-    if (SE_NUMAPPROX(cy - g.max1, 0.0)) {
-        t1 = g.nEls1 - 1;
-    } else {
-        double out = (cy - g.min1) / g.dx1;
-        frac = modf(out, &integer);
-        t1 = (int)integer;
-        if (t1 > 0 && SE_NUMAPPROX(frac, 0.0)) t1--;
+        t = (int)integer;
+        if (t > 0 && SE_NUMAPPROX(frac, 0.0)) t--;
     }
     // A coordinate outside the domain (displacement beyond one period, or a
     // non-finite velocity) has no element in the reference either; clamp so
     // the gather stays inside the field arrays.
-    t0 = t0 < 0 ? 0 : (t0 >= g.nEls0 ? g.nEls0 - 1 : t0);
-    t1 = t1 < 0 ? 0 : (t1 >= g.nEls1 ? g.nEls1 - 1 : t1);
-    return t1 * g.nEls0 + t0;
+    return t < 0 ? 0 : (t >= l.nEls ? l.nEls - 1 : t);
+}
+__device__ __forceinline__ int get_el(const SLGeom& g, double cx, double cy) {
+    return get_el(line_of<0>(g, 1), cy) * g.nEls0 + get_el(line_of<0>(g, 0), cx);
 }
 
-// Advector::PeriodicUpdate, src/base/Advector.cpp:122-134
-__device__ __forceinline__ void wrap(const SLGeom& g, double& cx, double& cy) {
+// Advector::PeriodicUpdate, src/base/Advector.cpp:122-134, in one dimension
+__device__ __forceinline__ void wrap(const Line& l, double& c) {
 #pragma clang fp contract(off)
-    if (cx < g.min0) cx = g.per0 ? g.max0 - g.min0 + cx : g.min0;
-    if (cx > g.max0) cx = g.per0 ? g.min0 - g.max0 + cx : g.max0;
-    if (cy < g.min1) cy = g.per1 ? g.max1 - g.min1 + cy : g.min1;
-    if (cy > g.max1) cy = g.per1 ? g.min1 - g.max1 + cy : g.max1;
+    if (c < l.min) c = l.per ? l.max - l.min + c : l.min;
+    if (c > l.max) c = l.per ? l.min - l.max + c : l.max;
 }
 
 // The kernels take the order as a template argument NN (the launches
@@ -91,58 +117,207 @@ __device__ __forceinline__ int order(const SLGeom& g) {
     return NN ? NN : g.N;
 }
 
-// Jacobi::EvalDeriv (Jacobi.cpp:58-66) of P_N; its powers of x share one
-// log (pow_int_at: each power the same bits as pow(x, i - 1))
+// Jacobi::EvalDeriv (Jacobi.cpp:58-66) of P_N; its powers of x share one log.
+// Between two GLL points no special case of pow arises (but |x| below 2^-60 at
+// odd orders): there the powers are free of branches and run side by side.
 template <int NN>
 __device__ __forceinline__ double pn_deriv(const SLGeom& g, double x) {
 #pragma clang fp contract(off)
-    const se_pow::PowBase b = se_pow::pow_base(x);
     double dp = 0.0;
-    for (int i = order<NN>(g); i >= 1; i -= 2) dp += g.pn[i] * i * se_pow::pow_int_at(b, i - 1);
+    if (se_pow::pow_plain(x)) {
+        double lo = 0.0, hi = 0.0;
+        if (order<NN>(g) > 2) hi = se_pow::log_hi_lo(se_pow::bits(x) & 0x7fffffffffffffffULL, &lo);
+        for (int i = order<NN>(g); i >= 1; i -= 2) dp += g.pn[i] * i * se_pow::pow_plain_at(x, hi, lo, i - 1);
+    } else {
+        const se_pow::PowBase b = se_pow::pow_base(x);
+#pragma unroll 1
+        for (int i = order<NN>(g); i >= 1; i -= 2) dp += g.pn[i] * i * se_pow::pow_int_at(b, i - 1);
+    }
     return dp;
 }
 
-// 1-D GLL cardinal functions at local coordinate x (Legendre::IsRoot and the
-// per-dimension factor of ShapeFuncsAtCoord, Legendre.cpp:145-169,291-305)
+// a / b, correctly rounded, for operands whose quotient and steps are far from
+// the limits of the exponent (or NaN): two Newton steps of the reciprocal, the
+// quotient and its remainder's correction (Markstein) without the scaling
+// around them.
+__device__ __forceinline__ double div_plain(double a, double b) {
+#pragma clang fp contract(off)
+    double r = __builtin_amdgcn_rcp(b);
+    r = fma(r, fma(-b, r, 1.0), r);
+    r = fma(r, fma(-b, r, 1.0), r);
+    const double q = a * r;
+    return fma(fma(-b, q, a), r, q);
+}
+
+// 1-D GLL cardinal functions at local coordinate x in [-1, 1] (Legendre::IsRoot
+// and the per-dimension factor of ShapeFuncsAtCoord, Legendre.cpp:145-169,
+// 291-305).  At least 1e-8 from every GLL point, 1 - x^2 is 2e-8 or more and
+// the divisor 1e-9 or more.
 template <int NN>
 __device__ __forceinline__ void cardinal(const SLGeom& g, double x, double (&L)[Ord<NN>::MAX + 1]) {
 #pragma clang fp contract(off)
     const int N = order<NN>(g);
     int root = -1;
-    for (int k = 0; k <= N; k++)
-        if (fabs(x - g.xk[k]) < 1.0e-8) {
-            root = k;
-            break;
-        }
+    for (int k = N; k >= 0; k--)
+        if (fabs(x - g.xk[k]) < 1.0e-8) root = k;
     if (root >= 0) {
         for (int j = 0; j <= N; j++) L[j] = (j == root) ? 1.0 : 0.0;
         return;
     }
     const double dpx = pn_deriv<NN>(g, x);
     for (int j = 0; j <= N; j++)
-        L[j] = -((1.0 - x * x) / (N * (N + 1) * g.pnx[j] * (x - g.xk[j]))) * dpx;
+        L[j] = -div_plain(1.0 - x * x, N * (N + 1) * g.pnx[j] * (x - g.xk[j])) * dpx;
 }
 
-// Field::InterpGlobal (Field.cpp:57-76) through Mesh::GlobalToLocal
-// (Mesh.cpp:163-177); vals node-major with ND dofs
+// Mesh::GlobalToLocal (Mesh.cpp:163-177) in one dimension; n0: the first node
+// of c's element along the dimension
+__device__ __forceinline__ double local_of(const Line& l, double c, int& n0) {
+#pragma clang fp contract(off)
+    const int e = get_el(l, c);
+    n0 = e * l.n0;
+    double x = (c - l.min - e * l.dx) * l.sc - 1.0;
+    if (x < -1.0) x = -1;
+    if (x > +1.0) x = +1;
+    return x;
+}
+
+// The element of a point whose coordinate in this lane's dimension is c
+struct Place {
+    double x;  // this dimension's local coordinate
+    int node;  // the element's first node
+};
+template <int NN>
+__device__ __forceinline__ Place place(const Line& l, double c) {
+    Place p;
+    int n0;
+    p.x = local_of(l, c, n0);
+    p.node = n0 + __builtin_amdgcn_mov_dpp(n0, kSwap, 0xf, 0xf, true);
+    return p;
+}
+
+// A point's weights: a lane evaluates its own dimension's, the pair exchanges
+template <int NN>
+struct Weights {
+    double x[Ord<NN>::MAX + 1], y[Ord<NN>::MAX + 1];
+    // hides the weights from the compiler before a further sum, whose products
+    // x y it would otherwise all keep from the one before
+    __device__ __forceinline__ void fresh() {
+        if (NN)
+#pragma unroll
+            for (int j = 0; j <= NN; j++) asm volatile("" : "+v"(y[j]));
+    }
+};
+template <int NN>
+__device__ __forceinline__ void weights_at(const SLGeom& g, const Place& p, Weights<NN>& w) {
+    double L[Ord<NN>::MAX + 1];
+    cardinal<NN>(g, p.x, L);
+    for (int j = 0; j <= order<NN>(g); j++) {
+        w.x[j] = quad<kEven>(L[j]);
+        w.y[j] = quad<kOdd>(L[j]);
+    }
+}
+
+// Field::InterpGlobal (Field.cpp:57-76) of one component per lane of a field of
+// nd components: a velocity's or a two-component field's own one (ND = 2), the
+// only one (ND = 1, both lanes) or component comp (ND = 0).  The cache's lookups bound the sums
+// on large meshes, so a lane reads 16 bytes at a time and the pair exchanges:
+// of two components the nodes of its parity, of one every other two nodes.
+// The first AHEAD rows of the element's nodes are read before the weights are
+// known, the others AHEAD rows before their use.
+struct __attribute__((aligned(8))) Two {
+    double a, b;
+};
+template <int NN, int ND>
+struct Rows {
+    static constexpr int AHEAD = NN > 6 ? 2 : 3, N1 = NN + 1;
+    static constexpr int NR = ND == 2 ? (N1 + 1) / 2 : ND == 1 ? (N1 + 3) / 4 : (N1 + 1) / 2;  // 16-byte reads a row
+    const double* p;
+    int nd, pitch, dim;
+    Two v[AHEAD][NR];
+
+    __device__ __forceinline__ void read(int jj) {
+        const double* r = p + jj * pitch;
+#pragma unroll
+        for (int k = 0; k < NR; k++) {
+            Two& t = v[jj % AHEAD][k];
+            if (ND == 2) {
+                t = *(const Two*)(r + 4 * k + (2 * k < NN ? 2 * dim : 0));
+            } else if (ND == 1) {
+                const int i0 = 4 * k < NN ? 4 * k : NN - 1, i1 = 4 * k + 2 < NN ? 4 * k + 2 : NN - 1;
+                t = *(const Two*)(r + (dim ? i1 : i0));
+            } else {
+                t.a = r[2 * k * nd];
+                if (2 * k < NN) t.b = r[(2 * k + 1) * nd];
+            }
+        }
+    }
+    __device__ __forceinline__ double value(int jj, int ii) const {
+        if (ND == 2) {  // lane 0 read the even nodes, lane 1 the odd ones
+            const Two& t = v[jj % AHEAD][ii / 2];
+            const double o = ii & 1 ? quad<kOdd>(t.a) : quad<kEven>(t.b);  // (with both lanes active)
+            return ii & 1 ? (dim ? t.b : o) : (dim ? o : t.a);
+        } else if (ND == 1) {
+            const Two& t = v[jj % AHEAD][ii / 4];
+            const int c = ii / 2 * 2, i0 = c < NN ? c : NN - 1;
+            return (ii & 2) ? quad<kOdd>(ii > i0 ? t.b : t.a) : quad<kEven>(ii > i0 ? t.b : t.a);
+        }
+        const Two& t = v[jj % AHEAD][ii / 2];
+        return ii & 1 ? t.b : t.a;
+    }
+    __device__ __forceinline__ Rows(const SLGeom& g, const Line& l, int node, const double* f, int nd_, int comp) {
+        nd = nd_;
+        dim = l.dim;
+        pitch = g.nv0 * nd;
+        p = f + (size_t)node * nd + (NN && ND ? 0 : comp);
+        if (NN)
+#pragma unroll
+            for (int jj = 0; jj < AHEAD && jj <= NN; jj++) read(jj);
+    }
+    __device__ __forceinline__ double sum(const SLGeom& g, const Weights<NN>& w) {
+#pragma clang fp contract(off)
+        double s = 0.0;
+        if (NN) {
+#pragma unroll
+            for (int jj = 0; jj <= NN; jj++) {
+#pragma unroll
+                for (int ii = 0; ii <= NN; ii++) s += w.x[ii] * w.y[jj] * value(jj, ii);
+                asm volatile("" : "+v"(s) : : "memory");  // the next rows' reads stay behind this row's sum
+                if (jj + AHEAD <= NN) read(jj + AHEAD);
+            }
+        } else {
+            for (int jj = 0; jj <= g.N; jj++)
+                for (int ii = 0; ii <= g.N; ii++)
+                    s += w.x[ii] * w.y[jj] * p[(size_t)jj * pitch + (size_t)ii * nd];
+        }
+        return s;
+    }
+};
+
+// this lane's component of a velocity at the point whose coordinate in its
+// dimension is c
+template <int NN>
+__device__ __forceinline__ double velocity_at(const SLGeom& g, const Line& l, double c, const double* __restrict__ vel,
+                                              Weights<NN>& w) {
+    const Place p = place<NN>(l, c);
+    Rows<NN, 2> r(g, l, p.node, vel, 2, l.dim);
+    weights_at<NN>(g, p, w);
+    return r.sum(g, w);
+}
+
+// Field::InterpGlobal at any point, one thread per point; vals node-major with
+// nd dofs
 template <int NN, int ND>
 __device__ __forceinline__ void interp_global(const SLGeom& g, const double* __restrict__ vals, int nd, double cx,
                                               double cy, double (&out)[ND]) {
 #pragma clang fp contract(off)
     const int N = order<NN>(g);
-    int el = get_el(g, cx, cy);
-    int ex = el % g.nEls0, ey = el / g.nEls0;
-    double lx = (cx - g.min0 - ex * g.dx0) * (2.0 / g.dx0) - 1.0;
-    double ly = (cy - g.min1 - ey * g.dx1) * (2.0 / g.dx1) - 1.0;
-    if (lx < -1.0) lx = -1;
-    if (lx > +1.0) lx = +1;
-    if (ly < -1.0) ly = -1;
-    if (ly > +1.0) ly = +1;
+    int nx, ny;
+    const double lx = local_of(line_of<NN>(g, 0), cx, nx), ly = local_of(line_of<NN>(g, 1), cy, ny);
     double Lx[Ord<NN>::MAX + 1], Ly[Ord<NN>::MAX + 1];
     cardinal<NN>(g, lx, Lx);
     cardinal<NN>(g, ly, Ly);
     for (int d = 0; d < ND; d++) out[d] = 0.0;
-    const int n0 = N * ey * g.nv0 + N * ex;
+    const int n0 = nx + ny;
 #pragma unroll 1
     for (int jj = 0; jj <= N; jj++)
         for (int ii = 0; ii <= N; ii++) {
@@ -150,40 +325,6 @@ __device__ __forceinline__ void interp_global(const SLGeom& g, const double* __r
             const double* v = &vals[(size_t)(n0 + jj * g.nv0 + ii) * nd];
             for (int d = 0; d < ND; d++)
                 if (d < nd) out[d] += Ni * v[d];
-        }
-}
-
-// interp_global of two node-major fields at one point (the weights computed
-// once): each output is summed exactly as interp_global sums it
-template <int NN, int NA, int NB>
-__device__ __forceinline__ void interp_global2(const SLGeom& g, const double* __restrict__ va, int na,
-                                               const double* __restrict__ vb, int nb, double cx, double cy,
-                                               double (&oa)[NA], double (&ob)[NB]) {
-#pragma clang fp contract(off)
-    const int N = order<NN>(g);
-    int el = get_el(g, cx, cy);
-    int ex = el % g.nEls0, ey = el / g.nEls0;
-    double lx = (cx - g.min0 - ex * g.dx0) * (2.0 / g.dx0) - 1.0;
-    double ly = (cy - g.min1 - ey * g.dx1) * (2.0 / g.dx1) - 1.0;
-    if (lx < -1.0) lx = -1;
-    if (lx > +1.0) lx = +1;
-    if (ly < -1.0) ly = -1;
-    if (ly > +1.0) ly = +1;
-    double Lx[Ord<NN>::MAX + 1], Ly[Ord<NN>::MAX + 1];
-    cardinal<NN>(g, lx, Lx);
-    cardinal<NN>(g, ly, Ly);
-    for (int d = 0; d < NA; d++) oa[d] = 0.0;
-    for (int d = 0; d < NB; d++) ob[d] = 0.0;
-    const int n0 = N * ey * g.nv0 + N * ex;
-#pragma unroll 1
-    for (int jj = 0; jj <= N; jj++)
-        for (int ii = 0; ii <= N; ii++) {
-            double Ni = Lx[ii] * Ly[jj];
-            const size_t node = (size_t)(n0 + jj * g.nv0 + ii);
-            for (int d = 0; d < NA; d++)
-                if (d < na) oa[d] += Ni * va[node * na + d];
-            for (int d = 0; d < NB; d++)
-                if (d < nb) ob[d] += Ni * vb[node * nb + d];
         }
 }
 
@@ -234,38 +375,67 @@ __device__ __forceinline__ void interp_bicubic(const SLGeom& g, const double* __
     interp_lagrange<ND>(cy, py, rows, out);
 }
 
+// The advected field's component of this lane -- and, of three, the last one
+__device__ __forceinline__ int component(const Line& l, int nd) { return l.dim < nd ? l.dim : nd - 1; }
+// the components at the point whose coordinate in this lane's dimension is c,
+// bicubic
+__device__ __forceinline__ void bicubic_at(const SLGeom& g, const Line& l, const double* __restrict__ q, int nd,
+                                           double c, double& a, double& b) {
+    const double o = quad<kSwap>(c);
+    double v[3];
+    interp_bicubic<3>(g, q, nd, l.dim ? o : c, l.dim ? c : o, v);
+    a = l.dim && nd > 1 ? v[1] : v[0];
+    b = v[2];
+}
+// the components by the weights of a place
 template <int NN, int ND>
-__device__ __forceinline__ void interp_any(const SLGeom& g, const double* __restrict__ vals, int nd, double cx,
-                                           double cy, double (&out)[ND]) {
-    if (g.cubic) interp_bicubic<ND>(g, vals, nd, cx, cy, out);
-    else interp_global<NN, ND>(g, vals, nd, cx, cy, out);
+__device__ __forceinline__ void advected_at(const SLGeom& g, const Line& l, double c, const double* __restrict__ q,
+                                            int nd, double& a, double& b) {
+    Weights<NN> w;
+    const Place p = place<NN>(l, c);
+    Rows<NN, ND> r(g, l, p.node, q, nd, component(l, nd));
+    weights_at<NN>(g, p, w);
+    a = r.sum(g, w);
+    b = 0.0;
+    if (ND == 0 && nd == 3) {
+        w.fresh();
+        b = Rows<NN, 0>(g, l, p.node, q, nd, 2).sum(g, w);
+    }
+}
+__device__ __forceinline__ void put_advected(const Line& l, int v, int nd, double a, double b,
+                                             double* __restrict__ qsl) {
+    if (l.dim < nd) qsl[(size_t)v * nd + l.dim] = a;
+    if (nd == 3 && l.dim == 0) qsl[(size_t)v * 3 + 2] = b;
 }
 
-// Advector::FirstOrder + IntegrateRK2 (Advector.cpp:136-148,181-201)
-template <int NN>
+// Advector::FirstOrder + IntegrateRK2 (Advector.cpp:136-148,181-201).  Bound by
+// latency: 29x17 order 5 22 -> 7.3 us, 32x32 order 6 29.5 -> 12 us with two lanes
+// per node, branch-free powers and unscaled divisions.
+template <int NN, int ND>
 __global__ __launch_bounds__(256) void k_sl_first(SLGeom g, const double* __restrict__ q, int nd,
                                                    const double* __restrict__ vel, double dt, double* __restrict__ qsl,
                                                    int32_t* __restrict__ dep) {
 #pragma clang fp contract(off)
-    int v = blockIdx.x * blockDim.x + threadIdx.x;
+    const int v = blockIdx.x * 128 + (threadIdx.x >> 1);
     if (v >= g.nv0 * g.nv1) return;
-    const double ox = g.X[v % g.nv0], oy = g.Y[v / g.nv0];
+    const Line l = line_of<NN>(g, threadIdx.x & 1);
+    const double o = l.dim ? g.Y[v / g.nv0] : g.X[v % g.nv0];
+    Weights<NN> w;
     // velocity at the origin: the origin is a GLL node, so InterpGlobal
     // returns the nodal value exactly (IsRoot selects a Kronecker delta)
-    double vel0[2];
-    interp_global<NN, 2>(g, vel, 2, ox, oy, vel0);
-    double hx = ox - 0.5 * dt * vel0[0];
-    double hy = oy - 0.5 * dt * vel0[1];
-    wrap(g, hx, hy);
-    double vh[2];
-    interp_global<NN, 2>(g, vel, 2, hx, hy, vh);
-    double cx = ox - dt * vh[0];
-    double cy = oy - dt * vh[1];
-    wrap(g, cx, cy);
-    double val[3];
-    interp_any<NN, 3>(g, q, nd, cx, cy, val);
-    for (int d = 0; d < nd; d++) qsl[(size_t)v * nd + d] = val[d];
-    if (dep) dep[v] = get_el(g, cx, cy);
+    double h = o - 0.5 * dt * velocity_at<NN>(g, l, o, vel, w);
+    wrap(l, h);
+    double c = o - dt * velocity_at<NN>(g, l, h, vel, w);
+    wrap(l, c);
+    double a, b;
+    if (ND < 0) bicubic_at(g, l, q, nd, c, a, b);
+    else advected_at<NN, ND>(g, l, c, q, nd, a, b);
+    put_advected(l, v, nd, a, b, qsl);
+    if (dep) {
+        const int e = get_el(l, c);
+        const int ey = __builtin_amdgcn_mov_dpp(e, kSwap, 0xf, 0xf, true);
+        if (l.dim == 0) dep[v] = ey * g.nEls0 + e;
+    }
 }
 
 // Advector::ExtrapolateVelocities (Advector.cpp:339-349)
@@ -280,43 +450,51 @@ __global__ void k_extrap(int n2, const double* __restrict__ vel, const double* _
     vmh[i] = 0.5 * a + 0.5 * b;
 }
 
-// Advector::SecondOrder (Advector.cpp:203-246).  Four waves per SIMD (at
-// most 128 VGPRs, ~160 bytes of spills) ran 7% faster than three (167 VGPRs):
-// the six gathers per node are latency-bound.
-template <int NN>
-__global__ __launch_bounds__(256, 4) void k_sl_second(SLGeom g, const double* __restrict__ q, const double* __restrict__ qp,
+// Advector::SecondOrder (Advector.cpp:203-246).  Four waves per SIMD (128
+// VGPRs, no spills; the bicubic form takes 256).  32x32 order 6 54 -> 19 us;
+// 96x96 order 6 135 -> 89 us: two thirds of it VALU issue (3300 instructions a
+// wave), the rest the cache's lookups of the gathers (126 us while a lane read 8
+// bytes at a time).
+template <int NN, int ND>
+__global__ __launch_bounds__(256, ND < 0 ? 2 : 4) void k_sl_second(SLGeom g, const double* __restrict__ q, const double* __restrict__ qp,
                                                     int nd, const double* __restrict__ vel,
                                                     const double* __restrict__ vp1, const double* __restrict__ vph,
                                                     const double* __restrict__ vmh, double dt,
                                                     double* __restrict__ qsl) {
 #pragma clang fp contract(off)
-    int v = blockIdx.x * blockDim.x + threadIdx.x;
+    const int v = blockIdx.x * 128 + (threadIdx.x >> 1);
     if (v >= g.nv0 * g.nv1) return;
-    const double ox = g.X[v % g.nv0], oy = g.Y[v / g.nv0];
-    double w[2];
-    interp_global<NN, 2>(g, vp1, 2, ox, oy, w);
-    double hx = ox - 0.5 * dt * w[0], hy = oy - 0.5 * dt * w[1];
-    wrap(g, hx, hy);
-    interp_global<NN, 2>(g, vph, 2, hx, hy, w);
-    double x1 = ox - dt * w[0], y1 = oy - dt * w[1];
-    wrap(g, x1, y1);
-    // the velocity and (GLL interpolation) the advected field at (x1, y1)
-    // share one set of weights
-    double p1[3], p2[3];
-    if (g.cubic) {
-        interp_global<NN, 2>(g, vel, 2, x1, y1, w);
-        interp_bicubic<3>(g, q, nd, x1, y1, p1);
+    const Line l = line_of<NN>(g, threadIdx.x & 1);
+    const double o = l.dim ? g.Y[v / g.nv0] : g.X[v % g.nv0];
+    Weights<NN> w;
+    double h = o - 0.5 * dt * velocity_at<NN>(g, l, o, vp1, w);
+    wrap(l, h);
+    double c = o - dt * velocity_at<NN>(g, l, h, vph, w);
+    wrap(l, c);
+    // the velocity and (GLL interpolation) the advected field at the first
+    // point share one set of weights
+    double a1, b1 = 0.0, a2, b2;
+    if (ND < 0) {
+        h = c - 0.5 * dt * velocity_at<NN>(g, l, c, vel, w);
+        bicubic_at(g, l, q, nd, c, a1, b1);
     } else {
-        interp_global2<NN, 2, 3>(g, vel, 2, q, nd, x1, y1, w, p1);
+        const Place p = place<NN>(l, c);
+        Rows<NN, 2> rv(g, l, p.node, vel, 2, l.dim);
+        weights_at<NN>(g, p, w);
+        h = c - 0.5 * dt * rv.sum(g, w);
+        w.fresh();
+        a1 = Rows<NN, ND>(g, l, p.node, q, nd, component(l, nd)).sum(g, w);
+        if (ND == 0 && nd == 3) {
+            w.fresh();
+            b1 = Rows<NN, 0>(g, l, p.node, q, nd, 2).sum(g, w);
+        }
     }
-    hx = x1 - 0.5 * dt * w[0];
-    hy = y1 - 0.5 * dt * w[1];
-    wrap(g, hx, hy);
-    interp_global<NN, 2>(g, vmh, 2, hx, hy, w);
-    double x2 = x1 - dt * w[0], y2 = y1 - dt * w[1];
-    wrap(g, x2, y2);
-    interp_any<NN, 3>(g, qp, nd, x2, y2, p2);
-    for (int d = 0; d < nd; d++) qsl[(size_t)v * nd + d] = 2.0 * p1[d] - 0.5 * p2[d];
+    wrap(l, h);
+    c -= dt * velocity_at<NN>(g, l, h, vmh, w);
+    wrap(l, c);
+    if (ND < 0) bicubic_at(g, l, qp, nd, c, a2, b2);
+    else advected_at<NN, ND>(g, l, c, qp, nd, a2, b2);
+    put_advected(l, v, nd, 2.0 * a1 - 0.5 * a2, 2.0 * b1 - 0.5 * b2, qsl);
 }
 
 // Field::PeriodicUpdate (Field.cpp:232-252) applied to the advected field
@@ -377,13 +555,12 @@ __global__ __launch_bounds__(256) void k_genvel(SLGeom g, const double* __restri
     double det = j00 * j11 - j01 * j10;
     double i00 = j11 / det, i11 = j00 / det, i01 = -j01 / det, i10 = -j10 / det;
     double g0 = 0.0, g1 = 0.0;
-    const int n0 = N * ey * g.nv0 + N * ex;
+    const double* p = psi + (N * ey * g.nv0 + N * ex);
     // the element's nodes (jj, ii) in row-major order; only row yi and
     // column xi can carry a non-zero shape-function derivative, so the walk
-    // visits those in the same order (the others were skipped anyway)
-    auto node = [&](int jj, int ii) {
-        double a0 = (jj == yi) ? g.D[xi * n1 + ii] : 0.0;  // GNx * Ny
-        double a1 = (ii == xi) ? g.D[yi * n1 + jj] : 0.0;  // Nx * GNy
+    // visits those in the same order (the others were skipped anyway).
+    // a0: GNx * Ny, a1: Nx * GNy
+    auto node = [&](double a0, double a1, double pv) {
         if (a0 == 0.0 && a1 == 0.0) return;
         double t0 = 0.0;
         t0 += a0 * i00;
@@ -391,13 +568,38 @@ __global__ __launch_bounds__(256) void k_genvel(SLGeom g, const double* __restri
         double t1 = 0.0;
         t1 += a0 * i10;
         t1 += a1 * i11;
-        double pv = psi[n0 + jj * g.nv0 + ii];
         g0 += t0 * pv;
         g1 += t1 * pv;
     };
-    for (int jj = 0; jj < yi; jj++) node(jj, xi);
-    for (int ii = 0; ii <= N; ii++) node(yi, ii);
-    for (int jj = yi + 1; jj <= N; jj++) node(jj, xi);
+    if (NN) {
+        // both lines of psi and of D before the first use (one node after the
+        // other the loads' latency was most of the time: 96x96 order 6 16 ->
+        // 12 us)
+        double pr[NN + 1], pc[NN + 1], dr[NN + 1], dc[NN + 1];
+#pragma unroll
+        for (int k = 0; k <= NN; k++) {
+            pr[k] = p[yi * g.nv0 + k];
+            pc[k] = p[k * g.nv0 + xi];
+            dr[k] = g.D[xi * n1 + k];
+            dc[k] = g.D[yi * n1 + k];
+        }
+#pragma unroll
+        for (int jj = 0; jj <= NN; jj++)
+            if (jj < yi) node(0.0, dc[jj], pc[jj]);
+        double dy = 0.0;  // D[yi][yi]
+#pragma unroll
+        for (int k = 0; k <= NN; k++)
+            if (k == yi) dy = dc[k];
+#pragma unroll
+        for (int ii = 0; ii <= NN; ii++) node(dr[ii], ii == xi ? dy : 0.0, pr[ii]);
+#pragma unroll
+        for (int jj = 0; jj <= NN; jj++)
+            if (jj > yi) node(0.0, dc[jj], pc[jj]);
+    } else {
+        for (int jj = 0; jj < yi; jj++) node(0.0, g.D[yi * n1 + jj], p[jj * g.nv0 + xi]);
+        for (int ii = 0; ii <= N; ii++) node(g.D[xi * n1 + ii], ii == xi ? g.D[yi * n1 + yi] : 0.0, p[yi * g.nv0 + ii]);
+        for (int jj = yi + 1; jj <= N; jj++) node(0.0, g.D[yi * n1 + jj], p[jj * g.nv0 + xi]);
+    }
     vel[2 * (size_t)v] = -1.0 * g1;
     vel[2 * (size_t)v + 1] = +1.0 * g0;
 }
@@ -450,6 +652,7 @@ SLGeom sl_geom(const se_mesh* m) {
 }
 
 int blocks_for(int n) { return (n + 255) / 256; }
+int pair_blocks(int n) { return n / 128 + (n % 128 != 0); }  // two lanes per node
 
 // KERNEL<N> for the orders 2..8, KERNEL<0> (the order read from the
 // geometry) for the others; 256 threads per workgroup
@@ -463,6 +666,24 @@ int blocks_for(int n) { return (n + 255) / 256; }
         case 7: hipLaunchKernelGGL(KERNEL<7>, GRID, dim3(256), 0, __VA_ARGS__); break; \
         case 8: hipLaunchKernelGGL(KERNEL<8>, GRID, dim3(256), 0, __VA_ARGS__); break; \
         default: hipLaunchKernelGGL(KERNEL<0>, GRID, dim3(256), 0, __VA_ARGS__); break; \
+    }
+
+// KERNEL<N, the advected components: 1, 2, else 0; -1: bicubic>
+#define SE_SL_ADV(KERNEL, N, GRID, ...)                                                                   \
+    if (g.cubic) hipLaunchKernelGGL((KERNEL<N, -1>), GRID, dim3(256), 0, __VA_ARGS__);                   \
+    else if (nd == 1) hipLaunchKernelGGL((KERNEL<N, 1>), GRID, dim3(256), 0, __VA_ARGS__);               \
+    else if (nd == 2) hipLaunchKernelGGL((KERNEL<N, 2>), GRID, dim3(256), 0, __VA_ARGS__);               \
+    else hipLaunchKernelGGL((KERNEL<N, 0>), GRID, dim3(256), 0, __VA_ARGS__)
+#define SE_SL_LAUNCH_ADV(KERNEL, N, GRID, ...)                        \
+    switch (N) {                                                      \
+        case 2: SE_SL_ADV(KERNEL, 2, GRID, __VA_ARGS__); break;       \
+        case 3: SE_SL_ADV(KERNEL, 3, GRID, __VA_ARGS__); break;       \
+        case 4: SE_SL_ADV(KERNEL, 4, GRID, __VA_ARGS__); break;       \
+        case 5: SE_SL_ADV(KERNEL, 5, GRID, __VA_ARGS__); break;       \
+        case 6: SE_SL_ADV(KERNEL, 6, GRID, __VA_ARGS__); break;       \
+        case 7: SE_SL_ADV(KERNEL, 7, GRID, __VA_ARGS__); break;       \
+        case 8: SE_SL_ADV(KERNEL, 8, GRID, __VA_ARGS__); break;       \
+        default: SE_SL_ADV(KERNEL, 0, GRID, __VA_ARGS__); break;      \
     }
 
 struct SLScratch {
@@ -484,7 +705,7 @@ extern "C" int se_sl_advect_dev(se_mesh* m, const double* d_q, int nd, const dou
              "bicubic advection (N < 3) needs at least 4 nodes per direction");
     SLGeom g = sl_geom(m);
     hipStream_t s = m->ctx->stream;
-    SE_SL_LAUNCH(k_sl_first, m->N, dim3(blocks_for(m->nV)), s, g, d_q, nd, d_vel, dt, d_qsl, d_dep);
+    SE_SL_LAUNCH_ADV(k_sl_first, m->N, dim3(pair_blocks(m->nV)), s, g, d_q, nd, d_vel, dt, d_qsl, d_dep);
     if (m->periodic[0] || m->periodic[1])
         hipLaunchKernelGGL(k_periodic_copy, dim3(blocks_for(m->nV)), dim3(256), 0, s, m->nVerts[0], m->nVerts[1],
                            m->periodic[0], m->periodic[1], nd, d_qsl);
@@ -514,7 +735,7 @@ int sl_second(se_mesh* m, const double* d_q, const double* d_qp, int nd, const d
     double* vph = vp1 + n2;
     double* vmh = vph + n2;
     hipLaunchKernelGGL(k_extrap, dim3(blocks_for((int)n2)), dim3(256), 0, s, (int)n2, d_vel, d_velp, vp1, vph, vmh);
-    SE_SL_LAUNCH(k_sl_second, m->N, dim3(blocks_for(m->nV)), s, g, d_q, d_qp, nd, d_vel, vp1, vph, vmh, dt, d_qsl);
+    SE_SL_LAUNCH_ADV(k_sl_second, m->N, dim3(pair_blocks(m->nV)), s, g, d_q, d_qp, nd, d_vel, vp1, vph, vmh, dt, d_qsl);
     if (m->periodic[0] || m->periodic[1])
         hipLaunchKernelGGL(k_periodic_copy, dim3(blocks_for(m->nV)), dim3(256), 0, s, m->nVerts[0], m->nVerts[1],
                            m->periodic[0], m->periodic[1], nd, d_qsl);
