@@ -1368,12 +1368,20 @@ struct FdmPlan {
     se_ctx* ctx = nullptr;
     std::vector<se_op*> ops;
     int prec = -1, cprec = -1;  // the transforms' precision: first application, corrections
-    DevBuf d_members, d_tasks;  // FbMember[count], GemmTask[4 count]
-    DevBuf d_tasks_c;           // GemmTask[4 count] of the corrections (cprec != prec)
-    DevBuf d_wtasks;            // WaveTask[count]; of a wave-form member the GemmTasks are unused
+    // The descriptors, packed in one device buffer and sent up in one copy from
+    // pinned memory: FbMember[count], WaveTask[count], ApplyMember[count] of
+    // p -> q and of x -> q, and, where a member's transforms are dense,
+    // GemmTask[4 count] and those of the corrections (cprec != prec).
+    DevBuf d_desc;
+    const FbMember* members = nullptr;
+    const WaveTask* wtasks = nullptr;  // of a wave-form member the GemmTasks are unused
+    const ApplyMember *ap = nullptr, *ax = nullptr;
+    const GemmTask *tasks = nullptr, *tasks_c = nullptr;
+    void* h_desc = nullptr;
+    size_t h_desc_cap = 0;
+    bool desc_pending = false;  // the copy may still read h_desc
     std::vector<WaveTask> h_wtasks;
     std::vector<FbMember> h_members;
-    DevBuf d_ap, d_ax;  // FP64 apply descriptors ApplyMember[count] (p -> q and x -> q)
     // Work lists of one member subset: (member, chunk) items of the vector
     // kernels, (member, tile) items of the transforms and of the apply,
     // and the member list, packed in one device
@@ -1388,6 +1396,7 @@ struct FdmPlan {
     // rewritten only after a stream synchronisation, and lists launched
     // together in one round come from different sets.
     struct Lists {
+        bool live = false;     // else only the buffer is kept, for the next subset
         std::vector<char> on;  // the member flags these lists were built for
         DevBuf d;
         const int2 *vwork = nullptr, *gwork = nullptr, *wave[4] = {}, *apply = nullptr;
@@ -1403,8 +1412,10 @@ struct FdmPlan {
         void* h = nullptr;           // pinned staging of an upload
         size_t hcap = 0;
         unsigned long long clock = 0;
-        void clear() {  // (no launch from these lists may be pending)
-            cache.clear();
+        // (a later launch or upload into the kept buffers follows those pending
+        // on the stream)
+        void clear() {
+            for (auto& e : cache) e->live = false;
             cur = nullptr;
         }
         ~ListSet() {
@@ -1429,12 +1440,13 @@ struct FdmPlan {
     // space): the start then stores no b, and a new f moves b with it (the
     // first pass-4 tasks and the A x descriptors name b)
     std::vector<char> b_alias;
-    std::vector<GemmTask> h_tasks;  // the host copy of d_tasks
+    std::vector<GemmTask> h_tasks, h_tasks_c;
     int desc_null = -1;
     double desc_rtol = 0.0;
 
     ~FdmPlan() {
         if (h_states) (void)hipHostFree(h_states);
+        if (h_desc) (void)hipHostFree(h_desc);
     }
 };
 
@@ -1514,7 +1526,7 @@ int plan_apply(FdmPlan* pl, int set, bool from_x, hipStream_t s, bool gated = fa
         // slot (four per CU) walks the list, instead of one per tile whose
         // dispatch alone costs ~20 us at the ensemble's 14 k tiles
         const int slots = std::max(8, 4 * pl->ctx->cu_count / 8 * 8);
-        launch_apply_any(mode, (from_x ? pl->d_ax : pl->d_ap).as<ApplyMember>(), L.apply, nw,
+        launch_apply_any(mode, from_x ? pl->ax : pl->ap, L.apply, nw,
                          gated ? std::min(nw, slots) : nw, s, gated ? 1 : 0);
     }
     // members with an SVV term: add it to the batched apply's result
@@ -1571,7 +1583,7 @@ int plan_lists(FdmPlan* pl, int set, const std::vector<char>& on, hipStream_t s)
     FdmPlan::ListSet& S = pl->sets[set];
     S.clock++;
     for (auto& e : S.cache)
-        if (e->on == on) {
+        if (e->live && e->on == on) {
             e->used = S.clock;
             S.cur = e.get();
             return SE_OK;
@@ -1616,14 +1628,21 @@ int plan_lists(FdmPlan* pl, int set, const std::vector<char>& on, hipStream_t s)
         SE_HIP(hipHostMalloc(&S.h, bytes, hipHostMallocDefault));
         S.hcap = bytes;
     }
-    if ((int)S.cache.size() >= FdmPlan::kListCache) {  // the least recently used subset makes room
-        SE_HIP(hipStreamSynchronize(s));                // no launch reads its lists
-        auto lru = std::min_element(S.cache.begin(), S.cache.end(),
-                                    [](const std::unique_ptr<FdmPlan::Lists>& a,
-                                       const std::unique_ptr<FdmPlan::Lists>& b) { return a->used < b->used; });
-        S.cache.erase(lru);
+    // a kept buffer no subset uses, a new one, or the least recently used subset's
+    FdmPlan::Lists* L = nullptr;
+    for (auto& e : S.cache)
+        if (!e->live && (!L || e->d.bytes > L->d.bytes)) L = e.get();
+    if (!L && (int)S.cache.size() < FdmPlan::kListCache) {
+        S.cache.emplace_back(new FdmPlan::Lists);
+        L = S.cache.back().get();
     }
-    std::unique_ptr<FdmPlan::Lists> L(new FdmPlan::Lists);
+    if (!L) {
+        SE_HIP(hipStreamSynchronize(s));  // no launch reads its lists
+        for (auto& e : S.cache)
+            if (!L || e->used < L->used) L = e.get();
+        L->live = false;
+    }
+    S.cur = nullptr;
     int rc = L->d.alloc(std::max<size_t>(bytes, sizeof(int2)));
     if (rc) return rc;
     char* h = static_cast<char*>(S.h);
@@ -1651,8 +1670,8 @@ int plan_lists(FdmPlan* pl, int set, const std::vector<char>& on, hipStream_t s)
     L->on = on;
     L->used = S.clock;
     if (bytes) SE_HIP(hipMemcpyAsync(L->d.ptr, S.h, bytes, hipMemcpyHostToDevice, s));
-    S.cur = L.get();
-    S.cache.push_back(std::move(L));
+    L->live = true;
+    S.cur = L;
     return SE_OK;
 }
 
@@ -1664,7 +1683,7 @@ int grid_of(size_t items, const se_ctx* c) {
 int plan_pass(FdmPlan* pl, int set, int pass, hipStream_t s, int skip = 0, int to_p = FDM_TO_Z, bool corr = false) {
     const FdmPlan::Lists& L = *pl->sets[set].cur;
     const bool c = corr && pl->cprec != pl->prec;
-    return launch_gemm(c ? pl->cprec : pl->prec, (c ? pl->d_tasks_c : pl->d_tasks).as<GemmTask>(), pass, L.gwork,
+    return launch_gemm(c ? pl->cprec : pl->prec, c ? pl->tasks_c : pl->tasks, pass, L.gwork,
                        L.n_gwork, s, skip, false, pass == 3 ? to_p : FDM_TO_Z);
 }
 
@@ -1672,7 +1691,7 @@ int plan_pass(FdmPlan* pl, int set, int pass, hipStream_t s, int skip = 0, int t
 int plan_wave(FdmPlan* pl, int set, int mode, hipStream_t s, int skip = 0, int to_p = FDM_TO_Z) {
     const FdmPlan::Lists& L = *pl->sets[set].cur;
     for (int k = mode == WAVE_Y ? 2 : 0, e = k + 2; k < e; k++) {
-        int rc = launch_wave(mode, k % 2 == 1, pl->d_wtasks.as<WaveTask>(), L.wave[k], L.n_wave[k], L.lds[k], s, skip,
+        int rc = launch_wave(mode, k % 2 == 1, pl->wtasks, L.wave[k], L.n_wave[k], L.lds[k], s, skip,
                              to_p);
         if (rc) return rc;
     }
@@ -1711,9 +1730,6 @@ int fdm_plan_set_members(FdmPlan* pl, int count, se_op* const* ops) {
         SE_HIP(hipHostMalloc((void**)&pl->h_states, sizeof(CgState) * count, hipHostMallocDefault));
         pl->h_cap = count;
     }
-    int rc = pl->d_members.alloc(sizeof(FbMember) * std::max(count, 1));
-    if (!rc) rc = pl->d_tasks.alloc(sizeof(GemmTask) * 4 * std::max(count, 1));
-    if (rc) return rc;
     pl->prec = -1;
     pl->cprec = -1;
     pl->desc_ok = false;
@@ -1732,9 +1748,12 @@ int fdm_plan_create(se_ctx* c, int count, se_op* const* ops, FdmPlan** out) {
 
 void fdm_plan_destroy(FdmPlan* pl) { delete pl; }
 
-// the FP64 apply descriptors: A p (+ p.q partials) and
-// A x (or, fused, the true residual), with each member's current iterate
-int upload_apply_descriptors(FdmPlan* pl, hipStream_t s) {
+// The descriptors' upload: the members, their transforms and their FP64
+// applies, A p (+ p.q partials) and A x (or, fused, the true residual), with
+// each member's current iterate.  One copy from pinned memory: a request
+// server re-members its plans as requests come and go, and six pageable copies
+// (each staged by the runtime) held its GPU idle for longer than the solve.
+int upload_descriptors(FdmPlan* pl, hipStream_t s) {
     std::vector<ApplyMember> ap, ax;
     for (size_t i = 0; i < pl->ops.size(); i++) {
         se_op* op = pl->ops[i];
@@ -1758,13 +1777,47 @@ int upload_apply_descriptors(FdmPlan* pl, hipStream_t s) {
         }
         ax.push_back(A);
     }
-    if (ap.empty()) return SE_OK;
-    int rc = pl->d_ap.alloc(sizeof(ApplyMember) * ap.size());
-    if (!rc) rc = pl->d_ax.alloc(sizeof(ApplyMember) * ax.size());
+    const size_t count = pl->ops.size();
+    if (count == 0) return SE_OK;
+    bool dense = false;
+    for (const FbMember& M : pl->h_members) dense = dense || !M.wave;
+    size_t total = 0;
+    auto block = [&](size_t bytes) {
+        const size_t at = total;
+        total += (bytes + 63) / 64 * 64;
+        return at;
+    };
+    const size_t nt = dense ? pl->h_tasks.size() : 0, nc = dense ? pl->h_tasks_c.size() : 0;
+    const size_t om = block(sizeof(FbMember) * count), ow = block(sizeof(WaveTask) * count);
+    const size_t op = block(sizeof(ApplyMember) * count), ox = block(sizeof(ApplyMember) * count);
+    const size_t ot = block(sizeof(GemmTask) * nt), oc = block(sizeof(GemmTask) * nc);
+    int rc = pl->d_desc.alloc(total);
     if (rc) return rc;
-    SE_HIP(hipMemcpyAsync(pl->d_ap.ptr, ap.data(), sizeof(ApplyMember) * ap.size(), hipMemcpyHostToDevice, s));
-    SE_HIP(hipMemcpyAsync(pl->d_ax.ptr, ax.data(), sizeof(ApplyMember) * ax.size(), hipMemcpyHostToDevice, s));
-    SE_HIP(hipStreamSynchronize(s));  // the host vectors go out of scope
+    if (pl->desc_pending || total > pl->h_desc_cap) SE_HIP(hipStreamSynchronize(s));
+    pl->desc_pending = false;
+    if (total > pl->h_desc_cap) {
+        if (pl->h_desc) (void)hipHostFree(pl->h_desc);
+        pl->h_desc = nullptr;
+        pl->h_desc_cap = 0;
+        SE_HIP(hipHostMalloc(&pl->h_desc, total, hipHostMallocDefault));
+        pl->h_desc_cap = total;
+    }
+    char* h = static_cast<char*>(pl->h_desc);
+    const char* d = pl->d_desc.as<char>();
+    std::memcpy(h + om, pl->h_members.data(), sizeof(FbMember) * count);
+    std::memcpy(h + ow, pl->h_wtasks.data(), sizeof(WaveTask) * count);
+    std::memcpy(h + op, ap.data(), sizeof(ApplyMember) * count);
+    std::memcpy(h + ox, ax.data(), sizeof(ApplyMember) * count);
+    if (nt) std::memcpy(h + ot, pl->h_tasks.data(), sizeof(GemmTask) * nt);
+    if (nc) std::memcpy(h + oc, pl->h_tasks_c.data(), sizeof(GemmTask) * nc);
+    pl->members = reinterpret_cast<const FbMember*>(d + om);
+    pl->wtasks = reinterpret_cast<const WaveTask*>(d + ow);
+    pl->ap = reinterpret_cast<const ApplyMember*>(d + op);
+    pl->ax = reinterpret_cast<const ApplyMember*>(d + ox);
+    pl->tasks = nt ? reinterpret_cast<const GemmTask*>(d + ot) : nullptr;
+    pl->tasks_c = nc ? reinterpret_cast<const GemmTask*>(d + oc) : nullptr;
+    pl->desc_pending = true;
+    SE_HIP(hipMemcpyAsync(pl->d_desc.ptr, h, total, hipMemcpyHostToDevice, s));
     return SE_OK;
 }
 
@@ -1792,7 +1845,7 @@ int fdm_plan_solve(FdmPlan* pl, const double* const* d_f, double* const* d_x, co
     const bool reuse = pl->desc_ok && pl->prec == prec && pl->cprec == cprec && pl->desc_null == null &&
                        pl->desc_rtol == o.rtol;
     if (reuse) {
-        bool changed = false, moved = false, bmoved = false;
+        bool changed = false;
         for (int i = 0; i < count; i++) {
             FbMember& M = pl->h_members[i];
             if (M.f != d_f[i] || M.xo != d_x[i]) {
@@ -1800,28 +1853,19 @@ int fdm_plan_solve(FdmPlan* pl, const double* const* d_f, double* const* d_x, co
                     M.b = const_cast<double*>(d_f[i]);  // read only: b is f
                     pl->h_tasks[4 * (size_t)i + 3].b = M.b;
                     pl->h_wtasks[i].b = M.b;
-                    bmoved = true;
                 }
                 M.f = d_f[i];
                 M.xo = d_x[i];
-                double* x = iterate_of(pl, i, d_f, d_x);
-                moved = moved || x != M.x;
-                M.x = x;
+                M.x = iterate_of(pl, i, d_f, d_x);
                 changed = true;
             }
         }
-        if (changed && count > 0)
-            SE_HIP(hipMemcpyAsync(pl->d_members.ptr, pl->h_members.data(), sizeof(FbMember) * count,
-                                  hipMemcpyHostToDevice, s));
-        if (bmoved) {
-            SE_HIP(hipMemcpyAsync(pl->d_tasks.ptr, pl->h_tasks.data(), sizeof(GemmTask) * 4 * count,
-                                  hipMemcpyHostToDevice, s));
-            SE_HIP(hipMemcpyAsync(pl->d_wtasks.ptr, pl->h_wtasks.data(), sizeof(WaveTask) * count,
-                                  hipMemcpyHostToDevice, s));
-        }
-        if (moved || bmoved) {  // the A x descriptors name the iterates and b
-            int e = upload_apply_descriptors(pl, s);
-            if (e) return e;
+        if (changed) {  // the applies name the iterates and b too
+            int e = upload_descriptors(pl, s);
+            if (e) {
+                pl->desc_ok = false;
+                return e;
+            }
         }
     } else {
         {
@@ -1829,15 +1873,9 @@ int fdm_plan_solve(FdmPlan* pl, const double* const* d_f, double* const* d_x, co
             if (rc) return rc;
         }
         pl->h_members.assign(count, FbMember{});
-        std::vector<GemmTask> tasks(4 * (size_t)count), tasks_c(cprec != prec ? 4 * (size_t)count : 0);
-        if (cprec != prec) {
-            int e = pl->d_tasks_c.alloc(sizeof(GemmTask) * 4 * std::max(count, 1));
-            if (e) return e;
-        }
-        {
-            int e = pl->d_wtasks.alloc(sizeof(WaveTask) * std::max(count, 1));
-            if (e) return e;
-        }
+        std::vector<GemmTask>&tasks = pl->h_tasks, &tasks_c = pl->h_tasks_c;
+        tasks.assign(4 * (size_t)count, GemmTask{});
+        tasks_c.assign(cprec != prec ? 4 * (size_t)count : 0, GemmTask{});
         pl->h_wtasks.assign(count, WaveTask{});
         pl->any_svv = false;
         for (se_op* op : pl->ops) pl->any_svv = pl->any_svv || op->svv_mN != 0;
@@ -1912,22 +1950,9 @@ int fdm_plan_solve(FdmPlan* pl, const double* const* d_f, double* const* d_x, co
                 }
             }
         }
-        int rc = SE_OK;
-        if (count > 0) {
-            SE_HIP(hipMemcpyAsync(pl->d_members.ptr, pl->h_members.data(), sizeof(FbMember) * count, hipMemcpyHostToDevice,
-                                  s));
-            SE_HIP(hipMemcpyAsync(pl->d_tasks.ptr, tasks.data(), sizeof(GemmTask) * 4 * count, hipMemcpyHostToDevice, s));
-            pl->h_tasks = tasks;
-            SE_HIP(hipMemcpyAsync(pl->d_wtasks.ptr, pl->h_wtasks.data(), sizeof(WaveTask) * count,
-                                  hipMemcpyHostToDevice, s));
-            if (cprec != prec)
-                SE_HIP(hipMemcpyAsync(pl->d_tasks_c.ptr, tasks_c.data(), sizeof(GemmTask) * 4 * count,
-                                      hipMemcpyHostToDevice, s));
-        }
         pl->prec = prec;
         pl->cprec = cprec;
-        // FP64 apply descriptors
-        rc = upload_apply_descriptors(pl, s);
+        int rc = upload_descriptors(pl, s);
         if (rc) return rc;
         for (auto& L : pl->sets) L.clear();  // new descriptors: new lists
         pl->desc_ok = true;
@@ -1942,10 +1967,11 @@ int fdm_plan_solve(FdmPlan* pl, const double* const* d_f, double* const* d_x, co
         h.status = CG_RUNNING;
         pl->h_states[i] = h;
     }
-    const FbMember* Ms = pl->d_members.as<FbMember>();
+    const FbMember* Ms = pl->members;
     auto pull = [&]() -> int {
         SE_HIP(hipMemcpyAsync(pl->h_states, pl->d_states.ptr, sizeof(CgState) * count, hipMemcpyDeviceToHost, s));
         SE_HIP(hipStreamSynchronize(s));
+        pl->desc_pending = false;
         return SE_OK;
     };
     auto vlaunch = [&](int set, void (*k)(const FbMember*, const int2*, int)) {
