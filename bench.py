@@ -217,18 +217,32 @@ def pc_code(a, prec_name, fdm_default=False):
     return se_amd.PC_JACOBI
 
 
-def fdm_roofline(pr, prec_name, kernel):
-    """pr: per-pass us / flops of the FDM transforms and us / bytes of the FP64 apply."""
-    us, fl = sum(pr["us_pass"]), sum(pr["flops_pass"])
-    ach = fl / (us * 1e-6) / 1e12
-    peak = MFMA_PEAK_TFLOPS[prec_name]
+def fdm_roofline(pr, prec_name):
+    """pr: us / flops of the FDM's four 1-D transforms and us / bytes of the FP64
+    apply.  BF16 transforms are four launches of the dense GEMM, bound by the
+    matrix cores.  The others run as plane waves over the elements in FP64, in
+    three launches -- x, both transforms of y (half of its time in each of two
+    entries), and back in x -- each of which reads and writes the unknowns once."""
     apply_gbs = pr["bytes_apply"] / (pr["us_apply"] * 1e-6) / 1e9
-    return {"kernel": kernel, "bound": "mfma", "achieved": ach, "peak": peak, "unit": "TFLOP/s",
-            "frac": ach / peak, "traffic": None, "us_per_launch": us / 4.0, "flops_per_launch": fl / 4.0,
-            "passes": [{"us": u, "flops": f, "tflops": f / (u * 1e-6) / 1e12} for u, f in zip(pr["us_pass"],
-                                                                                             pr["flops_pass"])],
-            "fp64_apply": {"us_per_launch": pr["us_apply"], "bytes_per_launch": pr["bytes_apply"],
-                           "achieved_gbs": apply_gbs, "frac_hbm": apply_gbs / HBM_PEAK_GBS}}
+    ps = list(zip(pr["us_pass"], pr["flops_pass"]))
+    wave = prec_name != "bf16_ir"
+    if wave:
+        ps = [ps[0], (ps[1][0] + ps[2][0], ps[1][1] + ps[2][1]), ps[3]]
+    us, fl = sum(u for u, _ in ps), sum(f for _, f in ps)
+    tflops = fl / (us * 1e-6) / 1e12
+    out = {"traffic": None, "us_per_launch": us / len(ps), "flops_per_launch": fl / len(ps),
+           "passes": [{"us": u, "flops": f, "tflops": f / (u * 1e-6) / 1e12} for u, f in ps],
+           "fp64_apply": {"us_per_launch": pr["us_apply"], "bytes_per_launch": pr["bytes_apply"],
+                          "achieved_gbs": apply_gbs, "frac_hbm": apply_gbs / HBM_PEAK_GBS}}
+    if wave:
+        ach = pr["bytes_apply"] * len(ps) / (us * 1e-6) / 1e9
+        out.update(kernel="k_fdm_wave", bound="hbm", achieved=ach, peak=HBM_PEAK_GBS, unit="GB/s",
+                   frac=ach / HBM_PEAK_GBS, bytes_per_launch=pr["bytes_apply"], mfma_tflops=tflops,
+                   mfma_frac=tflops / MFMA_PEAK_TFLOPS["fp64"])
+    else:
+        out.update(kernel="k_fdm_gemm<%s>" % GEMM_T[prec_name], bound="mfma", achieved=tflops,
+                   peak=MFMA_PEAK_TFLOPS[prec_name], unit="TFLOP/s", frac=tflops / MFMA_PEAK_TFLOPS[prec_name])
+    return out
 
 
 def run_ensemble(a, prec_name):
@@ -271,10 +285,11 @@ def run_ensemble(a, prec_name):
     value = ntot / (ms * 1e-3) / 1e9
     T = GEMM_T[prec_name]
     if pc == se_amd.PC_FDM:
-        # dominant kernel: the FDM transforms on the matrix cores (four passes
+        # dominant kernel: the FDM transforms on the matrix cores (each launch
         # over all members, timed back to back after the last solve)
-        roof = fdm_roofline(b.fdm_probe(reps=a.probe_reps), prec_name, "k_fdm_gemm<%s>" % T)
-        roof["traffic"] = pmc_traffic(roof, "k_fdm_gemm__ensemble_512_%s_pmc.md" % prec_name.split("_")[0])
+        roof = fdm_roofline(b.fdm_probe(reps=a.probe_reps), prec_name)
+        roof["traffic"] = pmc_traffic(roof, "%s__ensemble_512_%s_pmc.md" % (roof["kernel"].split("<")[0],
+                                                                            prec_name.split("_")[0]))
     else:
         # dominant kernel: the direction + separable operator kernel of the
         # largest order group (the probe continues the last solve's recurrences)
@@ -413,7 +428,7 @@ def run_single(a, prec_name):
               "all_converged": ok, "n_iter_per_s": m.n * info["iters"] / (ms * 1e-3), "wall_s_timed": t_wall}
     T = GEMM_T[prec_name]
     if pc == se_amd.PC_FDM:
-        roof = fdm_roofline(h.fdm_probe(reps=a.probe_reps), prec_name, "k_fdm_gemm<%s>" % T)
+        roof = fdm_roofline(h.fdm_probe(reps=a.probe_reps), prec_name)
     elif prec == se_amd.PREC_FP64:
         # dominant kernel: the FP64 operator apply, timed on its stream
         for _ in range(5):

@@ -1613,7 +1613,7 @@ int plan_lists(FdmPlan* pl, int set, const std::vector<char>& on, hipStream_t s)
         }
         xcd_interleave(ids, tiles, cost, cls, apply);
     }
-    // packed: vector items, transform items, per-order apply items (int2), member list (int)
+    // packed: vector items, transform items, apply items (int2), member list (int)
     size_t n2 = vwork.size() + gwork.size();
     for (const auto& w : wave) n2 += w.size();
     n2 += apply.size();

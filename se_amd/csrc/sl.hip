@@ -219,11 +219,11 @@ __device__ __forceinline__ void weights_at(const SLGeom& g, const Place& p, Weig
 
 // Field::InterpGlobal (Field.cpp:57-76) of one component per lane of a field of
 // nd components: a velocity's or a two-component field's own one (ND = 2), the
-// only one (ND = 1, both lanes) or component comp (ND = 0).  The cache's lookups bound the sums
-// on large meshes, so a lane reads 16 bytes at a time and the pair exchanges:
-// of two components the nodes of its parity, of one every other two nodes.
-// The first AHEAD rows of the element's nodes are read before the weights are
-// known, the others AHEAD rows before their use.
+// only one (ND = 1, both lanes) or component comp (ND = 0).  The cache's
+// lookups bound the sums on large meshes, so a lane reads 16 bytes at a time
+// and the pair exchanges: of two components the nodes of its parity, of one
+// every other two nodes.  The first AHEAD rows of the element's nodes are read
+// before the weights are known, the others AHEAD rows before their use.
 struct __attribute__((aligned(8))) Two {
     double a, b;
 };
