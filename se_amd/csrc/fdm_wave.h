@@ -83,6 +83,16 @@ __host__ __device__ inline size_t wave_lds(int N, int E, int E16, int LD) {
     return ((size_t)(kWavePad + E16) * LD + 16 + (wave_long(E) ? 0 : N * N * E16)) * sizeof(double);
 }
 
+// The thread, hidden from the compiler: each item derives its indices anew.
+// Kept over the loop of items (of every order's N x N product) they spilled 14
+// registers, and on the ensemble's short lines the scratch lines written back
+// were more than the data (512 members 3060 -> 3000 us, 24 channels 227 -> 223).
+__device__ __forceinline__ int wave_tid() {
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    return tid;
+}
+
 // U <- F U (FWD: slots -> phases, else phases -> slots): NQ output tiles of this
 // wave, all K steps.  Operands of zero stand where a block has fewer rows than
 // its tiles; the LDS rows they meet hold finite values (other blocks' or
@@ -144,7 +154,7 @@ __device__ __forceinline__ void wave_product(const WaveDim& d, const double* U, 
 // before the product (behind the lines' loads, the N x N matrices).
 template <bool FWD, int NA>
 __device__ __forceinline__ void wave_ahead(const WaveDim& d, WaveTiles<NA>& w) {
-    const int l = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l = wave_tid() & 63, wv = __builtin_amdgcn_readfirstlane(wave_tid() >> 6);
     const int nt = FWD ? d.nf : d.nb;
     typedef const __attribute__((address_space(4))) WaveTile ctile;  // (uniform: scalar loads)
     ctile* tab = (ctile*)(FWD ? d.tf : d.tb);
@@ -163,7 +173,7 @@ __device__ __forceinline__ void wave_ahead(const WaveDim& d, WaveTiles<NA>& w) {
 template <bool FWD, int NA>
 __device__ __forceinline__ void wave_matrix(double* U, const WaveDim& d, const WaveTiles<NA>& w) {
     constexpr bool LONG = NA > 4;
-    const int l = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l = wave_tid() & 63, wv = __builtin_amdgcn_readfirstlane(wave_tid() >> 6);
     const int nt = FWD ? d.nf : d.nb;
     const WaveTile(&t)[NA] = w.t;
     wave_f64x4 acc[NA];
@@ -199,10 +209,10 @@ __device__ __forceinline__ void wave_matrix(double* U, const WaveDim& d, const W
 // U's rows outside the phases, and the parts of a slot without an element:
 // operands of zero meet them
 __device__ __forceinline__ void wave_pad(const WaveDim& d, double* U, bool slots) {
-    for (int k = threadIdx.x; k < kWavePad * d.LD; k += kWaveT) U[k - kWavePad * d.LD] = 0.0;
-    for (int k = d.E * d.LD + threadIdx.x; k < d.E16 * d.LD; k += kWaveT) U[k] = 0.0;
+    for (int k = wave_tid(); k < kWavePad * d.LD; k += kWaveT) U[k - kWavePad * d.LD] = 0.0;
+    for (int k = d.E * d.LD + wave_tid(); k < d.E16 * d.LD; k += kWaveT) U[k] = 0.0;
     if (slots && d.ne < d.E)
-        for (int k = (1 << d.logR) + threadIdx.x; k < d.LD; k += kWaveT) U[(d.E - 1) * d.LD + k] = 0.0;
+        for (int k = (1 << d.logR) + wave_tid(); k < d.LD; k += kWaveT) U[(d.E - 1) * d.LD + k] = 0.0;
 }
 
 constexpr double kR2 = 0.70710678118654752440;
@@ -214,8 +224,8 @@ constexpr double kR2 = 0.70710678118654752440;
 template <int B, typename AT>
 __device__ __forceinline__ void wave_load(const WaveTask& t, const WaveDim& d, double* U, bool ok, AT&& at) {
     const int N = t.N, P1 = 1 + t.nS, mul = 65536 / P1 + 1;  // (exact below 2^16 / P1)
-    const int cnt = (d.n0 * P1) << d.logR, r = threadIdx.x & ((1 << d.logR) - 1);
-    for (int k0 = threadIdx.x; k0 < cnt; k0 += B * kWaveT) {
+    const int cnt = (d.n0 * P1) << d.logR, r = wave_tid() & ((1 << d.logR) - 1);
+    for (int k0 = wave_tid(); k0 < cnt; k0 += B * kWaveT) {
         double v[B][4];
         int s_[B], i_[B], m_[B];
 #pragma unroll
@@ -261,10 +271,10 @@ __device__ __forceinline__ void wave_load(const WaveTask& t, const WaveDim& d, d
 template <bool TO_U, typename OUT>
 __device__ __forceinline__ void wave_unfold(const WaveTask& t, const WaveDim& d, double* U, bool ok, OUT&& out) {
     const int N = t.N, P1 = 1 + t.nS, mul = 65536 / P1 + 1;
-    const int cnt = (d.n0 * P1) << d.logR, r = threadIdx.x & ((1 << d.logR) - 1);
+    const int cnt = (d.n0 * P1) << d.logR, r = wave_tid() & ((1 << d.logR) - 1);
     if (!ok && !TO_U) return;
 #pragma unroll 2
-    for (int k = threadIdx.x; k < cnt; k += kWaveT) {
+    for (int k = wave_tid(); k < cnt; k += kWaveT) {
         const int idx = k >> d.logR, s = (idx * mul) >> 16, i = idx - s * P1, A = t.nS << d.logR;
         const bool pair = i > 0 && 2 * i != N;
         if (i > 0 && (s >= d.n1 || s >= d.ne)) continue;
@@ -303,7 +313,7 @@ __device__ __forceinline__ double wave_modes(const WaveTask& t, const WaveDim& d
                                              int item) {
     double rz = 0.0;  // WAVE_Y: this thread's part of r.z
     const int R = 1 << d.logR, h = d.logR - 1;
-    for (int k = threadIdx.x; k < d.E << h; k += kWaveT) {
+    for (int k = wave_tid(); k < d.E << h; k += kWaveT) {
         const int r = 2 * (k & ((1 << h) - 1)), c = k >> h;
         double2* u = reinterpret_cast<double2*>(U + c * d.LD + r);
         auto f = [&](int p, int j) -> double {
@@ -403,7 +413,7 @@ __device__ __forceinline__ void wave_block(const WaveTask& t, const WaveDim& d, 
     const unsigned mul = (1u << 24) / w + 1;            // (exact: below 2^13 units, w at most 32)
     SE_GLOBAL wave_d2* T = (SE_GLOBAL wave_d2*)gview(t.t1) + (size_t)item * cnt;
 #pragma unroll 4
-    for (int k = threadIdx.x; k < cnt; k += kWaveT) {
+    for (int k = wave_tid(); k < cnt; k += kWaveT) {
         const int c = (int)(((unsigned long long)k * mul) >> 24), j = k - c * w;
         wave_d2* u = (wave_d2*)(U + c * d.LD) + j;
         if (OUT) T[k] = *u;
@@ -423,7 +433,7 @@ __global__ __launch_bounds__(kWaveT, LONG ? 2 : 4) void k_fdm_wave(const WaveTas
         if (skip && wave_skip(t)) continue;
         const WaveDim& d = MODE == WAVE_Y ? t.y : t.x;
         const int R = 1 << d.logR, lgx = t.x.logR, Rx = 1 << lgx, nMx = t.x.E * t.N;
-        const int line = (it.y << d.logR) + (threadIdx.x & (R - 1));  // this thread's line
+        const int line = (it.y << d.logR) + (wave_tid() & (R - 1));  // this thread's line
         const bool ok = line < (MODE == WAVE_Y ? nMx : t.y.n);
         // unknown J of column `line` in T1
         auto in_t1 = [&](int J) { return (((size_t)(J >> lgx) * nMx + line) << lgx) + (J & (Rx - 1)); };
@@ -446,7 +456,7 @@ __global__ __launch_bounds__(kWaveT, LONG ? 2 : 4) void k_fdm_wave(const WaveTas
         if (!LONG) {
             const SE_GLOBAL wave_d2* f = (const SE_GLOBAL wave_d2*)gview(d.phi);
 #pragma unroll 4
-            for (int k = threadIdx.x; k < (t.N * t.N * d.E16) >> 1; k += kWaveT) ((wave_d2*)Phi)[k] = f[k];
+            for (int k = wave_tid(); k < (t.N * t.N * d.E16) >> 1; k += kWaveT) ((wave_d2*)Phi)[k] = f[k];
         }
         __syncthreads();
         if (MODE != WAVE_XB) wave_matrix<true>(U, d, tiles);
@@ -470,7 +480,7 @@ __global__ __launch_bounds__(kWaveT, LONG ? 2 : 4) void k_fdm_wave(const WaveTas
             wave_unfold<true>(t, d, U, ok, [](int, double) {});
             __syncthreads();
             SE_GLOBAL double* Z = gview(to_p != 0 ? t.p : t.z) + (size_t)line * d.n;
-            const int N = t.N, mul = 65536 / N + 1, r = threadIdx.x & (R - 1);  // (nodes below 2^16 / N)
+            const int N = t.N, mul = 65536 / N + 1, r = wave_tid() & (R - 1);  // (nodes below 2^16 / N)
             auto node = [&](int I) {
                 const int a = I + d.off, e = (a * mul) >> 16, i = a - e * N;
                 const int p = i <= t.nS ? i : t.nS + N - i, s = i == 0 ? e - d.vs : e;
@@ -479,14 +489,14 @@ __global__ __launch_bounds__(kWaveT, LONG ? 2 : 4) void k_fdm_wave(const WaveTas
             if (!t.null_space) {
                 if (ok) {
 #pragma unroll 8
-                    for (int I = threadIdx.x >> d.logR; I < d.n; I += kWaveT >> d.logR) Z[I] = node(I);
+                    for (int I = wave_tid() >> d.logR; I < d.n; I += kWaveT >> d.logR) Z[I] = node(I);
                 }
                 continue;
             }
             const SE_GLOBAL double* Rs = gview(to_p == 2 ? t.b : t.r) + (size_t)line * d.n;
             double sz = 0.0, sr = 0.0;
 #pragma unroll 4
-            for (int I = threadIdx.x >> d.logR; I < d.n; I += kWaveT >> d.logR)
+            for (int I = wave_tid() >> d.logR; I < d.n; I += kWaveT >> d.logR)
                 if (ok) {
                     const double v = node(I);
                     Z[I] = v;
