@@ -402,10 +402,23 @@ __device__ __forceinline__ void advected_at(const SLGeom& g, const Line& l, doub
         b = Rows<NN, 0>(g, l, p.node, q, nd, 2).sum(g, w);
     }
 }
-__device__ __forceinline__ void put_advected(const Line& l, int v, int nd, double a, double b,
+// Stores node v's value, with Field::PeriodicUpdate (Field.cpp:232-252): the
+// first line's nodes of a periodic dimension also store their duplicates on the
+// last line, whose own values go nowhere (a launch of its own cost 4 us and an
+// edge after each step).
+__device__ __forceinline__ void put_advected(const SLGeom& g, const Line& l, int v, int nd, double a, double b,
                                              double* __restrict__ qsl) {
-    if (l.dim < nd) qsl[(size_t)v * nd + l.dim] = a;
-    if (nd == 3 && l.dim == 0) qsl[(size_t)v * 3 + 2] = b;
+    const int J = v / g.nv0, I = v - J * g.nv0;
+    if ((g.per0 && I == g.nv0 - 1) || (g.per1 && J == g.nv1 - 1)) return;
+    auto put = [&](int at) {
+        if (l.dim < nd) qsl[(size_t)at * nd + l.dim] = a;
+        if (nd == 3 && l.dim == 0) qsl[(size_t)at * 3 + 2] = b;
+    };
+    const int x = g.per0 && I == 0 ? g.nv0 - 1 : 0, y = g.per1 && J == 0 ? (g.nv1 - 1) * g.nv0 : 0;
+    put(v);
+    if (x) put(v + x);
+    if (y) put(v + y);
+    if (x && y) put(v + x + y);
 }
 
 // Advector::FirstOrder + IntegrateRK2 (Advector.cpp:136-148,181-201).  Bound by
@@ -430,7 +443,7 @@ __global__ __launch_bounds__(256) void k_sl_first(SLGeom g, const double* __rest
     double a, b;
     if (ND < 0) bicubic_at(g, l, q, nd, c, a, b);
     else advected_at<NN, ND>(g, l, c, q, nd, a, b);
-    put_advected(l, v, nd, a, b, qsl);
+    put_advected(g, l, v, nd, a, b, qsl);
     if (dep) {
         const int e = get_el(l, c);
         const int ey = __builtin_amdgcn_mov_dpp(e, kSwap, 0xf, 0xf, true);
@@ -494,18 +507,7 @@ __global__ __launch_bounds__(256, ND < 0 ? 2 : 4) void k_sl_second(SLGeom g, con
     wrap(l, c);
     if (ND < 0) bicubic_at(g, l, qp, nd, c, a2, b2);
     else advected_at<NN, ND>(g, l, c, qp, nd, a2, b2);
-    put_advected(l, v, nd, 2.0 * a1 - 0.5 * a2, 2.0 * b1 - 0.5 * b2, qsl);
-}
-
-// Field::PeriodicUpdate (Field.cpp:232-252) applied to the advected field
-__global__ void k_periodic_copy(int nv0, int nv1, int per0, int per1, int nd, double* __restrict__ f) {
-    int v = blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= nv0 * nv1) return;
-    int I = v % nv0, J = v / nv0;
-    bool dupI = per0 && I == nv0 - 1, dupJ = per1 && J == nv1 - 1;
-    if (!dupI && !dupJ) return;
-    int src = (dupJ ? 0 : J) * nv0 + (dupI ? 0 : I);
-    for (int d = 0; d < nd; d++) f[(size_t)v * nd + d] = f[(size_t)src * nd + d];
+    put_advected(g, l, v, nd, 2.0 * a1 - 0.5 * a2, 2.0 * b1 - 0.5 * b2, qsl);
 }
 
 // Field::InterpGlobal (mode GLL) or Advector::Interpolate (mode BICUBIC) at
@@ -706,9 +708,6 @@ extern "C" int se_sl_advect_dev(se_mesh* m, const double* d_q, int nd, const dou
     SLGeom g = sl_geom(m);
     hipStream_t s = m->ctx->stream;
     SE_SL_LAUNCH_ADV(k_sl_first, m->N, dim3(pair_blocks(m->nV)), s, g, d_q, nd, d_vel, dt, d_qsl, d_dep);
-    if (m->periodic[0] || m->periodic[1])
-        hipLaunchKernelGGL(k_periodic_copy, dim3(blocks_for(m->nV)), dim3(256), 0, s, m->nVerts[0], m->nVerts[1],
-                           m->periodic[0], m->periodic[1], nd, d_qsl);
     SE_HIP(hipGetLastError());
     return SE_OK;
 }
@@ -736,9 +735,6 @@ int sl_second(se_mesh* m, const double* d_q, const double* d_qp, int nd, const d
     double* vmh = vph + n2;
     hipLaunchKernelGGL(k_extrap, dim3(blocks_for((int)n2)), dim3(256), 0, s, (int)n2, d_vel, d_velp, vp1, vph, vmh);
     SE_SL_LAUNCH_ADV(k_sl_second, m->N, dim3(pair_blocks(m->nV)), s, g, d_q, d_qp, nd, d_vel, vp1, vph, vmh, dt, d_qsl);
-    if (m->periodic[0] || m->periodic[1])
-        hipLaunchKernelGGL(k_periodic_copy, dim3(blocks_for(m->nV)), dim3(256), 0, s, m->nVerts[0], m->nVerts[1],
-                           m->periodic[0], m->periodic[1], nd, d_qsl);
     SE_HIP(hipGetLastError());
     return SE_OK;
 }
