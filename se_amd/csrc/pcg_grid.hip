@@ -626,8 +626,9 @@ std::mutex g_grid_busy[kDevices];  // one grid-wide solve per device at a time
 
 // The solve as one launch.  done = false: not of this form (too large for the
 // chip's LDS and registers, an SVV term, a recorded history), another such
-// solve is running on the device, or a wait ran out; nothing has been written
-// then and the caller solves it launch by launch.
+// solve is running on the device, or a wait ran out; f is whole then (d_x may
+// hold part of a result: workgroups past the last sum have stored theirs) and
+// the caller solves it launch by launch.
 int pcg_grid(se_op* op, const double* d_f, double* d_x, const se_solve_opts& o, se_solve_info& info, bool& done) {
     done = false;
     se_mesh* m = op->mesh;
@@ -697,7 +698,11 @@ int pcg_grid(se_op* op, const double* d_f, double* d_x, const se_solve_opts& o, 
     if (hs->pad) return SE_OK;  // a wait ran out (the slots are cleared before the next use)
     op->grid_dirty = false;
     op->grid_turn ^= 1;
-    if (a.x != d_x) SE_HIP(hipMemcpyAsync(d_x, a.x, sizeof(double) * m->n, hipMemcpyDeviceToDevice, s));
+    if (a.x != d_x) {  // only now: a solve that gave up still needs f, which d_x is
+        SE_HIP(hipMemcpyAsync(d_x, a.x, sizeof(double) * m->n, hipMemcpyDeviceToDevice, s));
+        SE_HIP(hipEventRecord(c->ev1, s));
+        SE_HIP(hipEventSynchronize(c->ev1));
+    }
     float ms = 0.f;
     (void)hipEventElapsedTime(&ms, c->ev0, c->ev1);
     info.status = hs->status;
