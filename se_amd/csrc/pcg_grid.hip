@@ -36,11 +36,12 @@
 //
 // Waits are bounded: a workgroup whose partners do not arrive within `limit`
 // (workgroups that are not resident together) gives up, all leave, and the
-// caller runs the launch-per-phase solver instead.  At most one such launch
-// per device and process is in flight (pcg_grid), so two of them cannot hold
-// each other's workgroups out.
+// caller runs the launch-per-phase solver instead.  The solves of a process
+// share a device's CUs by turns (GridGate), so they cannot hold each other's
+// workgroups out.
 #include <algorithm>
 #include <cmath>
+#include <condition_variable>
 #include <cstdlib>
 #include <mutex>
 
@@ -619,14 +620,50 @@ int launch_grid_n(const GridArgs& a, const GridShape& sh, hipStream_t s) {
     return sh.T == 256 ? launch_grid<N, 256>(a, sh, s) : launch_grid<N, 576>(a, sh, s);
 }
 
+// The CUs of a device that the solves in flight from this process may need.  A
+// workgroup needs a CU at most, so the workgroups of a solve that was let in
+// are all resident once other kernels have drained.  A solve waits its turn:
+// going to the other solver where the device is taken would give it other
+// round-off, and so a result that depends on what runs beside it.
+struct GridGate {
+    std::mutex mu;
+    std::condition_variable cv;
+    unsigned long long next = 0, serving = 0;  // tickets: solves enter in order of arrival
+    int used = 0;
+    void enter(int cus, int all) {
+        std::unique_lock<std::mutex> lk(mu);
+        const unsigned long long t = next++;
+        cv.wait(lk, [&] { return t == serving && used + cus <= all; });
+        serving++;
+        used += cus;
+        cv.notify_all();
+    }
+    void leave(int cus) {
+        std::lock_guard<std::mutex> lk(mu);
+        used -= cus;
+        cv.notify_all();
+    }
+};
 constexpr int kDevices = 64;
-std::mutex g_grid_busy[kDevices];  // one grid-wide solve per device at a time
+GridGate g_gate[kDevices];
+// a solve's stay, from before its launch until its kernel has ended; a lone
+// workgroup waits for no other and needs none
+struct GridStay {
+    GridGate& gate;
+    int cus;
+    GridStay(GridGate& g, int n, int all) : gate(g), cus(n) {
+        if (cus > 1) gate.enter(cus, all);
+    }
+    ~GridStay() {
+        if (cus > 1) gate.leave(cus);
+    }
+};
 
 }  // namespace
 
 // The solve as one launch.  done = false: not of this form (too large for the
-// chip's LDS and registers, an SVV term, a recorded history), another such
-// solve is running on the device, or a wait ran out; f is whole then (d_x may
+// chip's LDS and registers, an SVV term, a recorded history), or a wait ran
+// out; f is whole then (d_x may
 // hold part of a result: workgroups past the last sum have stored theirs) and
 // the caller solves it launch by launch.
 int pcg_grid(se_op* op, const double* d_f, double* d_x, const se_solve_opts& o, se_solve_info& info, bool& done) {
@@ -636,8 +673,6 @@ int pcg_grid(se_op* op, const double* d_f, double* d_x, const se_solve_opts& o, 
     if (o.history || op->svv_mN > 0 || m->n < 1 || c->device >= kDevices) return SE_OK;
     GridShape sh;
     if (!grid_shape(m, c->cu_count, sh)) return SE_OK;
-    std::unique_lock<std::mutex> lk(g_grid_busy[c->device], std::try_to_lock);
-    if (!lk.owns_lock()) return SE_OK;
     hipStream_t s = c->stream;
     // two regions of slots: a solve uses one and its workgroups empty theirs
     // in the other for the next solve
@@ -679,6 +714,7 @@ int pcg_grid(se_op* op, const double* d_f, double* d_x, const se_solve_opts& o, 
     // SE_GRID_WAIT (seconds): another limit; 0: no wait at all
     const char* wait = getenv("SE_GRID_WAIT");
     a.limit = (u64)((wait ? atof(wait) : kWaitLimit) * 1e8);
+    GridStay stay(g_gate[c->device], sh.G, c->cu_count);
     SE_HIP(hipEventRecord(c->ev0, s));
     int rc = SE_ERR_UNSUPPORTED;
     switch (m->N) {

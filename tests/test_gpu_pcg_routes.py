@@ -1,5 +1,6 @@
 """FP64 Jacobi-PCG solves around the one-launch solver (pcg_grid.hip): what a
 caller sees of a solve does not depend on how it is called or what runs beside it."""
+import threading
 
 import numpy as np
 import pytest
@@ -33,3 +34,31 @@ def test_in_place_solve_is_complete(gpu_ctx):
         assert done and np.array_equal(got, want)
     h.close()
     m.close()
+
+
+def test_solves_beside_other_threads(gpu_ctx):
+    """Solves of three contexts on one device from three threads, more workgroups
+    in all than CUs: each solve the bits it has alone."""
+    ctxs = [gpu_ctx, se_amd.Context(0), se_amd.Context(0)]
+    probs = [problem(c, n, N, seed=N) for c, n, N in zip(ctxs, ((100, 100), (48, 40), (9, 7)), (8, 6, 5))]
+    alone = [h.pcg(f) for _, h, f in probs]
+    got = [[] for _ in probs]
+    start = threading.Barrier(len(probs))
+
+    def work(i):
+        start.wait()
+        for _ in range(4):
+            got[i].append(probs[i][1].pcg(probs[i][2])[0])
+
+    ts = [threading.Thread(target=work, args=(i,)) for i in range(len(probs))]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    for (x, info), xs in zip(alone, got):
+        assert info["status"] == 0 and len(xs) == 4 and all(np.array_equal(x, y) for y in xs)
+    for m, h, _ in probs:
+        h.close()
+        m.close()
+    for c in ctxs[1:]:
+        c.close()
