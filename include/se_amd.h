@@ -97,6 +97,11 @@ void* se_ctx_stream(se_ctx* ctx); /* the context's hipStream_t */
  * counterpart in the reference: the yardstick for the HBM byte counters and
  * the attainable copy bandwidth in the measurements. */
 int se_ctx_copy_probe(se_ctx* ctx, size_t bytes, int reps, double* us);
+/* FP64 Jacobi-PCG solves of this context so far that ran as one launch, and
+ * such launches that gave up a wait for workgroups that were not resident
+ * (their solves then ran launch per phase).  No counterpart in the reference:
+ * shows which of the two solvers a call took. */
+int se_ctx_solver_counts(const se_ctx* ctx, int64_t* one_launch, int64_t* gave_up);
 
 /* ---- mesh and global numbering --------------------------------------------
  * [ref: Mesh::Mesh src/base/Mesh.cpp:17-84 with elType "legendre";

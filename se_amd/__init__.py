@@ -129,6 +129,7 @@ def lib():
             "se_ctx_synchronize": (i, [vp]),
             "se_ctx_stream": (vp, [vp]),
             "se_ctx_copy_probe": (i, [vp, C.c_size_t, i, C.POINTER(d)]),
+            "se_ctx_solver_counts": (i, [vp, C.POINTER(C.c_int64), C.POINTER(C.c_int64)]),
             "se_mesh_create": (i, [vp, _I, i, _D, _D, _I, _I, pvp]),
             "se_mesh_destroy": (i, [vp]),
             "se_mesh_get_info": (i, [vp, C.POINTER(MeshInfo)]),
@@ -369,6 +370,13 @@ class Context:
         us = C.c_double()
         check(lib().se_ctx_copy_probe(self.h, int(nbytes), int(reps), C.byref(us)), "se_ctx_copy_probe")
         return us.value
+
+    def solver_counts(self):
+        """(FP64 Jacobi-PCG solves so far that ran as one launch, launches that
+        gave up a wait and left their solve to the launch-per-phase solver)."""
+        a, b = C.c_int64(), C.c_int64()
+        check(lib().se_ctx_solver_counts(self.h, C.byref(a), C.byref(b)), "se_ctx_solver_counts")
+        return a.value, b.value
 
     def close(self):
         """Destroy the context and, first, everything still alive that was

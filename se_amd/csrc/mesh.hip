@@ -314,6 +314,13 @@ extern "C" int se_ctx_copy_probe(se_ctx* c, size_t bytes, int reps, double* us) 
     return SE_OK;
 }
 
+extern "C" int se_ctx_solver_counts(const se_ctx* c, int64_t* one_launch, int64_t* gave_up) {
+    SE_CHECK(c && one_launch && gave_up, SE_ERR_ARG, "se_ctx_solver_counts: NULL argument");
+    *one_launch = c->grid_solves;
+    *gave_up = c->grid_gave_up;
+    return SE_OK;
+}
+
 // ---------------------------------------------------------------------------
 // C ABI: mesh
 // ---------------------------------------------------------------------------

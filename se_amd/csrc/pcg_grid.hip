@@ -40,6 +40,7 @@
 // share a device's CUs by turns (GridGate), so they cannot hold each other's
 // workgroups out.
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <condition_variable>
 #include <cstdlib>
@@ -606,18 +607,38 @@ bool grid_shape(const se_mesh* m, int cu, GridShape& best) {
     return cost < HUGE_VAL;
 }
 
+constexpr int kDevices = 64;
+
+// The kernel may have kLdsMax of LDS and then fits a CU: set and asked once per
+// kernel and device.
 template <int N, int T>
-int launch_grid(const GridArgs& a, const GridShape& sh, hipStream_t s) {
-    auto k = k_pcg_grid<N, T>;
-    SE_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
-                               (int)kLdsMax));
-    hipLaunchKernelGGL(k, dim3(sh.G), dim3(T), sh.lds, s, a);
+bool grid_usable(int device) {
+    static std::atomic<signed char> known[kDevices];  // 1: usable, -1: not
+    signed char k = known[device].load();
+    if (k == 0) {
+        const void* f = reinterpret_cast<const void*>(k_pcg_grid<N, T>);
+        int blocks = 0;
+        const bool ok =
+            hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsMax) == hipSuccess &&
+            hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, f, T, kLdsMax) == hipSuccess && blocks >= 1;
+        if (!ok) (void)hipGetLastError();
+        k = ok ? 1 : -1;
+        known[device].store(k);
+    }
+    return k > 0;
+}
+
+// SE_ERR_UNSUPPORTED: not launched
+template <int N, int T>
+int launch_grid(const GridArgs& a, const GridShape& sh, int device, hipStream_t s) {
+    if (!grid_usable<N, T>(device)) return SE_ERR_UNSUPPORTED;
+    hipLaunchKernelGGL((k_pcg_grid<N, T>), dim3(sh.G), dim3(T), sh.lds, s, a);
     return SE_OK;
 }
 
 template <int N>
-int launch_grid_n(const GridArgs& a, const GridShape& sh, hipStream_t s) {
-    return sh.T == 256 ? launch_grid<N, 256>(a, sh, s) : launch_grid<N, 576>(a, sh, s);
+int launch_grid_n(const GridArgs& a, const GridShape& sh, int device, hipStream_t s) {
+    return sh.T == 256 ? launch_grid<N, 256>(a, sh, device, s) : launch_grid<N, 576>(a, sh, device, s);
 }
 
 // The CUs of a device that the solves in flight from this process may need.  A
@@ -643,8 +664,21 @@ struct GridGate {
         used -= cus;
         cv.notify_all();
     }
+    // Waits that ran out in a row (another process on the device, masked CUs).
+    // One may be a passing kernel's.  From the second on the next solves, 16 and
+    // twice as many each time, are left to the other solver: a try costs the
+    // whole wait, 0.1 s, ten times an ordinary solve.
+    int strikes = 0, skip = 0;
+    bool leaves_out() {
+        std::lock_guard<std::mutex> lk(mu);
+        return skip > 0 && skip--;
+    }
+    void ended(bool well) {
+        std::lock_guard<std::mutex> lk(mu);
+        strikes = well ? 0 : strikes + 1;
+        if (strikes > 1) skip = 16 << std::min(strikes - 2, 16);
+    }
 };
-constexpr int kDevices = 64;
 GridGate g_gate[kDevices];
 // a solve's stay, from before its launch until its kernel has ended; a lone
 // workgroup waits for no other and needs none
@@ -663,7 +697,7 @@ struct GridStay {
 
 // The solve as one launch.  done = false: not of this form (too large for the
 // chip's LDS and registers, an SVV term, a recorded history), or a wait ran
-// out; f is whole then (d_x may
+// out, now or in solves before it; f is whole then (d_x may
 // hold part of a result: workgroups past the last sum have stored theirs) and
 // the caller solves it launch by launch.
 int pcg_grid(se_op* op, const double* d_f, double* d_x, const se_solve_opts& o, se_solve_info& info, bool& done) {
@@ -673,6 +707,8 @@ int pcg_grid(se_op* op, const double* d_f, double* d_x, const se_solve_opts& o, 
     if (o.history || op->svv_mN > 0 || m->n < 1 || c->device >= kDevices) return SE_OK;
     GridShape sh;
     if (!grid_shape(m, c->cu_count, sh)) return SE_OK;
+    GridGate& gate = g_gate[c->device];
+    if (sh.G > 1 && gate.leaves_out()) return SE_OK;
     hipStream_t s = c->stream;
     // two regions of slots: a solve uses one and its workgroups empty theirs
     // in the other for the next solve
@@ -714,24 +750,29 @@ int pcg_grid(se_op* op, const double* d_f, double* d_x, const se_solve_opts& o, 
     // SE_GRID_WAIT (seconds): another limit; 0: no wait at all
     const char* wait = getenv("SE_GRID_WAIT");
     a.limit = (u64)((wait ? atof(wait) : kWaitLimit) * 1e8);
-    GridStay stay(g_gate[c->device], sh.G, c->cu_count);
+    GridStay stay(gate, sh.G, c->cu_count);
     SE_HIP(hipEventRecord(c->ev0, s));
     int rc = SE_ERR_UNSUPPORTED;
     switch (m->N) {
-        case 2: rc = launch_grid_n<2>(a, sh, s); break;
-        case 3: rc = launch_grid_n<3>(a, sh, s); break;
-        case 4: rc = launch_grid_n<4>(a, sh, s); break;
-        case 5: rc = launch_grid_n<5>(a, sh, s); break;
-        case 6: rc = launch_grid_n<6>(a, sh, s); break;
-        case 7: rc = launch_grid_n<7>(a, sh, s); break;
-        case 8: rc = launch_grid_n<8>(a, sh, s); break;
-        default: return SE_OK;
+        case 2: rc = launch_grid_n<2>(a, sh, c->device, s); break;
+        case 3: rc = launch_grid_n<3>(a, sh, c->device, s); break;
+        case 4: rc = launch_grid_n<4>(a, sh, c->device, s); break;
+        case 5: rc = launch_grid_n<5>(a, sh, c->device, s); break;
+        case 6: rc = launch_grid_n<6>(a, sh, c->device, s); break;
+        case 7: rc = launch_grid_n<7>(a, sh, c->device, s); break;
+        case 8: rc = launch_grid_n<8>(a, sh, c->device, s); break;
+        default: break;
     }
-    if (rc) return rc;
+    if (rc == SE_ERR_UNSUPPORTED) return SE_OK;
     SE_HIP(hipGetLastError());
     SE_HIP(hipEventRecord(c->ev1, s));
     SE_HIP(hipEventSynchronize(c->ev1));
-    if (hs->pad) return SE_OK;  // a wait ran out (the slots are cleared before the next use)
+    if (sh.G > 1) gate.ended(!hs->pad);
+    if (hs->pad) {  // a wait ran out (the slots are cleared before the next use)
+        c->grid_gave_up++;
+        return SE_OK;
+    }
+    c->grid_solves++;
     op->grid_dirty = false;
     op->grid_turn ^= 1;
     if (a.x != d_x) {  // only now: a solve that gave up still needs f, which d_x is

@@ -81,6 +81,9 @@ struct se_ctx {
     // launch shapes chosen by the batched solver's autotuner, per
     // (order, log2 of the work items): later batches of that shape reuse them
     std::map<std::pair<int, int>, int> tuned_grid;
+    // FP64 Jacobi-PCG solves that ran as one launch, and such launches whose
+    // wait ran out
+    int64_t grid_solves = 0, grid_gave_up = 0;
 };
 
 struct se_mesh {

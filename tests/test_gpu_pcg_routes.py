@@ -1,5 +1,6 @@
 """FP64 Jacobi-PCG solves around the one-launch solver (pcg_grid.hip): what a
 caller sees of a solve does not depend on how it is called or what runs beside it."""
+import os
 import threading
 
 import numpy as np
@@ -62,3 +63,39 @@ def test_solves_beside_other_threads(gpu_ctx):
         m.close()
     for c in ctxs[1:]:
         c.close()
+
+
+def test_waits_that_ran_out_in_a_row_are_remembered(gpu_ctx):
+    """One give-up changes nothing for the solve after it; from the second in a
+    row on, 16 solves and then twice as many go straight to the other solver.
+    A lone workgroup never waits."""
+    m, h, f = problem(gpu_ctx, (24, 24), 6)
+    m1, h1, f1 = problem(gpu_ctx, (4, 4), 4)
+
+    def solve(n=1):
+        a = gpu_ctx.solver_counts()
+        for _ in range(n):
+            h.pcg(f, maxit=2)
+        b = gpu_ctx.solver_counts()
+        return b[0] - a[0], b[1] - a[1]
+
+    assert solve() == (1, 0)
+    os.environ["SE_GRID_WAIT"] = "0"
+    try:
+        assert solve() == (0, 1)
+        del os.environ["SE_GRID_WAIT"]
+        assert solve() == (1, 0)
+        os.environ["SE_GRID_WAIT"] = "0"
+        assert solve(2) == (0, 2)
+        assert solve(16) == (0, 0)
+        assert solve() == (0, 1)
+    finally:
+        os.environ.pop("SE_GRID_WAIT", None)
+    assert solve(31) == (0, 0)
+    a = gpu_ctx.solver_counts()
+    h1.pcg(f1)
+    assert gpu_ctx.solver_counts() == (a[0] + 1, a[1])
+    assert solve() == (0, 0)
+    assert solve(2) == (2, 0)
+    for o in (h, m, h1, m1):
+        o.close()
