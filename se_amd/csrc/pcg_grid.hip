@@ -434,6 +434,7 @@ __global__ __launch_bounds__(T) void k_pcg_grid(GridArgs g) {
     int iter = 0, guard = 0, status = CG_RUNNING;
     if (bb == 0.0) status = 0;
     else if (!(bb - bb == 0.0) || !(v[1] - v[1] == 0.0)) status = 3;
+    if (status == 3 && bb - bb == 0.0) tt = bb;  // (x = 0: the residual is b)
     if (mu != 0.0 && status == CG_RUNNING) {
 #pragma unroll
         for (int k = 0; k < NL; k++)

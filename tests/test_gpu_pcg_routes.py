@@ -99,3 +99,16 @@ def test_waits_that_ran_out_in_a_row_are_remembered(gpu_ctx):
     assert solve(2) == (2, 0)
     for o in (h, m, h1, m1):
         o.close()
+
+
+def test_overflow_at_the_start_reports_its_residual(gpu_ctx):
+    """b.b finite, r.z not: x = 0 and the relative residual is 1, in either solver."""
+    m = se_amd.Mesh(gpu_ctx, (12, 10), 4, (0.0, 0.0), (1.0, 1.0), XPER, (1, 1, 0, 0))
+    h = se_amd.Helm(m, 0.0, 1e-12, se_amd.DETJ_PHYSICAL)
+    f = 1e151 * np.random.default_rng(1).standard_normal(m.n)
+    for kw in ({}, dict(history=True, maxit=50)):
+        x, i = h.pcg(f, **kw)
+        assert i["status"] == se_amd.SOLVE_NONFINITE and i["iters"] == 0 and not x.any()
+        assert abs(i["true_rel_residual"] - 1.0) <= 1e-12
+    h.close()
+    m.close()
