@@ -218,11 +218,12 @@ int se_helm_apply_inner(se_op* op, int precision, const float* x, float* y, int*
  * Uses the operator's solver work vectors. */
 int se_helm_apply_fdm(se_op* op, int precision, const double* r, double* z);
 /* Measurement hook (no counterpart in the reference): after an FDM solve of
- * op, times `reps` back-to-back launches of each of the four transform
- * passes (the first with its residual pack) and of the FP64 operator apply,
- * with HIP events on the context stream: us_pass[4], flops_pass[4] (2 M N K
- * per member, padded sizes), us_apply, bytes_apply (16 B per unknown, 4 B
- * per field node). */
+ * op, times `reps` back-to-back launches of each of the four 1-D transforms
+ * and of the FP64 operator apply, with HIP events on the context stream:
+ * us_pass[4] (the plane-wave form does both transforms in y in one launch:
+ * half of its time each), flops_pass[4] (plane waves: 2 (E / 2 or E, + N) per
+ * unknown of a line of E elements; dense: 2 M N K, padded sizes), us_apply,
+ * bytes_apply (16 B per unknown). */
 int se_helm_fdm_probe(se_op* op, int reps, double* us_pass, double* flops_pass, double* us_apply,
                       double* bytes_apply);
 /* Measurement hook (no counterpart in the reference): after a mixed-precision

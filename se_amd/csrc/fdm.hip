@@ -2135,11 +2135,13 @@ int fdm_plan_solve(FdmPlan* pl, const double* const* d_f, double* const* d_x, co
 }
 
 // Measurement: after a solve of the plan, time `reps` back-to-back launches
-// of each transform pass over all members (pass 1 with its residual pack)
-// and of the FP64 operator apply, with HIP events on the context stream.
-// Per pass: microseconds per launch and flops per launch (2 M N K summed over
-// the members' padded sizes); the apply: microseconds and algorithmic bytes
-// (16 B per unknown for x and y).
+// of each of the four 1-D transforms over all members and of the FP64 operator
+// apply, with HIP events on the context stream.  A transform's time is that of
+// its wave kernel and its dense pass, where the plan has members of either form
+// (half of WAVE_Y's for each of the two in y).  Per transform: microseconds and
+// flops per launch, summed over the members (waves: wave_flops, dense: 2 M N K of
+// the padded sizes); the apply: microseconds and algorithmic bytes (16 B per
+// unknown for x and y).
 int fdm_plan_probe(FdmPlan* pl, int reps, double* us_pass, double* flops_pass, double* us_apply, double* bytes_apply) {
     SE_CHECK(pl->prec >= 0, SE_ERR_STATE, "FDM probe: run an FDM solve first");
     se_ctx* c = pl->ctx;
@@ -2148,43 +2150,41 @@ int fdm_plan_probe(FdmPlan* pl, int reps, double* us_pass, double* flops_pass, d
     std::vector<char> all(count, 1);
     int rc = plan_lists(pl, FdmPlan::SET_OTHER, all, s);
     if (rc) return rc;
-    // the four 1-D transforms; a wave kernel that does two counts half for each
-    const bool wave = count > 0 && pl->h_members[0].wave;
-    for (int pass = 0; pass < 4; pass++) {
-        const int mode = pass == 0 ? WAVE_X : (pass == 3 ? WAVE_XB : WAVE_Y);
-        auto once = [&]() {
-            return wave ? plan_wave(pl, FdmPlan::SET_OTHER, mode, s) : plan_pass(pl, FdmPlan::SET_OTHER, pass, s);
-        };
-        double fl = 0.0;
-        for (se_op* op : pl->ops) {
-            const double nP0 = op->fdm->nP0, nP1 = op->fdm->nP1;
-            fl += wave ? wave_flops(op, mode == WAVE_Y ? 1 : 0) : 2.0 * nP0 * nP1 * ((pass == 0 || pass == 3) ? nP0 : nP1);
-        }
-        flops_pass[pass] = fl;
-        rc = once();
-        if (rc) return rc;
+    auto time_of = [&](auto once, double& us) -> int {
+        int e = once();
+        if (e) return e;
         SE_HIP(hipEventRecord(c->ev0, s));
-        for (int r = 0; r < reps && !rc; r++) rc = once();
+        for (int r = 0; r < reps && !e; r++) e = once();
         SE_HIP(hipEventRecord(c->ev1, s));
         SE_HIP(hipEventSynchronize(c->ev1));
-        if (rc) return rc;
+        if (e) return e;
         float ms = 0.f;
         (void)hipEventElapsedTime(&ms, c->ev0, c->ev1);
-        us_pass[pass] = 1e3 * ms / reps * (wave && mode == WAVE_Y ? 0.5 : 1.0);
+        us = 1e3 * ms / reps;
+        return SE_OK;
+    };
+    bool wave = false, dense = false;
+    for (const FbMember& M : pl->h_members) (M.wave ? wave : dense) = true;
+    for (int pass = 0; pass < 4; pass++) {
+        const int mode = pass == 0 ? WAVE_X : (pass == 3 ? WAVE_XB : WAVE_Y);
+        double fl = 0.0, uw = 0.0, ud = 0.0;
+        for (int i = 0; i < count; i++) {
+            const se_op* op = pl->ops[i];
+            const double nP0 = op->fdm->nP0, nP1 = op->fdm->nP1;
+            fl += pl->h_members[i].wave ? wave_flops(op, mode == WAVE_Y ? 1 : 0)
+                                        : 2.0 * nP0 * nP1 * ((pass == 0 || pass == 3) ? nP0 : nP1);
+        }
+        flops_pass[pass] = fl;
+        if (wave) rc = time_of([&] { return plan_wave(pl, FdmPlan::SET_OTHER, mode, s); }, uw);
+        if (!rc && dense) rc = time_of([&] { return plan_pass(pl, FdmPlan::SET_OTHER, pass, s); }, ud);
+        if (rc) return rc;
+        us_pass[pass] = (mode == WAVE_Y ? 0.5 : 1.0) * uw + ud;
     }
     double by = 0.0;
     for (se_op* op : pl->ops) by += 16.0 * op->mesh->n;
     *bytes_apply = by;
-    rc = plan_apply(pl, FdmPlan::SET_OTHER, false, s);
+    rc = time_of([&] { return plan_apply(pl, FdmPlan::SET_OTHER, false, s); }, *us_apply);
     if (rc) return rc;
-    SE_HIP(hipEventRecord(c->ev0, s));
-    for (int r = 0; r < reps && !rc; r++) rc = plan_apply(pl, FdmPlan::SET_OTHER, false, s);
-    SE_HIP(hipEventRecord(c->ev1, s));
-    SE_HIP(hipEventSynchronize(c->ev1));
-    if (rc) return rc;
-    float ms = 0.f;
-    (void)hipEventElapsedTime(&ms, c->ev0, c->ev1);
-    *us_apply = 1e3 * ms / reps;
     SE_HIP(hipGetLastError());
     return SE_OK;
 }

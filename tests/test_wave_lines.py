@@ -54,3 +54,27 @@ def test_wave_inverse(gpu_ctx, ex, ey, N, per, bc):
     b.close()
     for o in (h, m, h2, m2):
         o.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("order", [(0, 1), (1, 0)])
+def test_probe_of_a_batch_of_both_forms(gpu_ctx, order):
+    """A wave-form member beside a dense one (a line of 257 elements): the probe
+    counts each with its own form's flops and times both."""
+    sizes = [((40, 12), 5), ((257, 2), 2)]
+    ms = [se_amd.Mesh(gpu_ctx, *sizes[k], (0.0, 0.0), (1.0, 1.0), (1, 0), (1, 1, 0, 0)) for k in order]
+    hs = [se_amd.Helm(m, 2.0, 1.0, se_amd.DETJ_PHYSICAL) for m in ms]
+    fs = [np.random.default_rng(k).standard_normal(m.n) for k, m in enumerate(ms)]
+    kw = dict(precision=se_amd.PREC_FP64, preconditioner=se_amd.PC_FDM)
+    flops = np.zeros(4)
+    for h, f in zip(hs, fs):
+        h.pcg(f, **kw)
+        flops += h.fdm_probe(reps=2)["flops_pass"]
+    b = se_amd.Batch(gpu_ctx, hs)
+    b.pcg(fs, **kw)
+    p = b.fdm_probe(reps=2)
+    assert np.array_equal(p["flops_pass"], flops)
+    assert min(p["us_pass"]) > 0.0 and p["us_apply"] > 0.0 and p["bytes_apply"] == 16.0 * sum(m.n for m in ms)
+    b.close()
+    for o in hs + ms:
+        o.close()
