@@ -30,6 +30,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstring>
 #include <map>
@@ -1111,19 +1112,38 @@ double wave_flops(const se_op* op, int axis) {
     return 2.0 * F->nU0 * F->nU1 * ((L.mirror[0] >= 0 ? 0.5 : 1.0) * L.E + L.N);
 }
 
+// The kernel may have the LDS of the largest line: set once per kernel and
+// device (set to each launch's own size, another thread could lower it between
+// a setting and its launch).
+constexpr size_t kWaveLdsMax = 116 * 1024;  // order 8, 128 elements
+template <int MODE, bool LONG>
+int wave_lds_limit() {
+    static std::atomic<bool> set[64];
+    int device = 0;
+    SE_HIP(hipGetDevice(&device));
+    if (device < 64 && set[device].load()) return SE_OK;
+    SE_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_fdm_wave<MODE, LONG>),
+                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)kWaveLdsMax));
+    if (device < 64) set[device].store(true);
+    return SE_OK;
+}
+
+template <int MODE, bool LONG>
+int launch_wave_t(const WaveTask* tasks, const int2* work, int nwork, size_t lds, hipStream_t s, int skip, int to_p) {
+    SE_CHECK(lds <= kWaveLdsMax, SE_ERR_STATE, "FDM: a line's block does not fit LDS");
+    int rc = wave_lds_limit<MODE, LONG>();
+    if (rc) return rc;
+    hipLaunchKernelGGL((k_fdm_wave<MODE, LONG>), dim3(nwork), dim3(kWaveT), lds, s, tasks, work, nwork, skip, to_p);
+    return SE_OK;
+}
+
 int launch_wave(int mode, bool lng, const WaveTask* tasks, const int2* work, int nwork, size_t lds, hipStream_t s,
                 int skip, int to_p) {
     if (nwork <= 0) return SE_OK;
-    auto go = [&](auto k) -> int {
-        if (lds > 64 * 1024)
-            SE_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       (int)lds));
-        hipLaunchKernelGGL(k, dim3(nwork), dim3(kWaveT), lds, s, tasks, work, nwork, skip, to_p);
-        return SE_OK;
-    };
-    if (mode == WAVE_X) return lng ? go(k_fdm_wave<WAVE_X, true>) : go(k_fdm_wave<WAVE_X, false>);
-    if (mode == WAVE_Y) return lng ? go(k_fdm_wave<WAVE_Y, true>) : go(k_fdm_wave<WAVE_Y, false>);
-    return lng ? go(k_fdm_wave<WAVE_XB, true>) : go(k_fdm_wave<WAVE_XB, false>);
+    auto go = [&](auto launch) { return launch(tasks, work, nwork, lds, s, skip, to_p); };
+    if (mode == WAVE_X) return lng ? go(launch_wave_t<WAVE_X, true>) : go(launch_wave_t<WAVE_X, false>);
+    if (mode == WAVE_Y) return lng ? go(launch_wave_t<WAVE_Y, true>) : go(launch_wave_t<WAVE_Y, false>);
+    return lng ? go(launch_wave_t<WAVE_XB, true>) : go(launch_wave_t<WAVE_XB, false>);
 }
 
 // FDM tables of op (FP64 part: eigenvectors, eigenvalues, mass factors and
