@@ -180,16 +180,22 @@ __device__ __forceinline__ void wave_matrix(double* U, const WaveDim& d, const W
 #pragma unroll
     for (int q = 0; q < NA; q++) acc[q] = wave_f64x4{0.0, 0.0, 0.0, 0.0};
     const int mine = (nt - wv + 7) >> 3;
-    if (LONG) {
-        wave_product<NA, NA, FWD>(d, U, w, acc, l);
-    } else {
-        switch (mine) {
-            case 0: break;
-            case 1: wave_product<1, NA, FWD>(d, U, w, acc, l); break;
-            case 2: wave_product<2, NA, FWD>(d, U, w, acc, l); break;
-            case 3: wave_product<3, NA, FWD>(d, U, w, acc, l); break;
-            default: wave_product<NA, NA, FWD>(d, U, w, acc, l); break;
-        }
+    // (a wave forms its own tiles only; 5 and 6 of the long lines' 7: at 256
+    // elements of order 2 a product of 7 for 4 cost a fifth of a solve)
+    switch (mine) {
+        case 0: break;
+        case 1: wave_product<1, NA, FWD>(d, U, w, acc, l); break;
+        case 2: wave_product<2, NA, FWD>(d, U, w, acc, l); break;
+        case 3: wave_product<3, NA, FWD>(d, U, w, acc, l); break;
+        default:
+            if constexpr (LONG) {
+                if (mine == 4) wave_product<4, NA, FWD>(d, U, w, acc, l);
+                else if (mine == 5) wave_product<5, NA, FWD>(d, U, w, acc, l);
+                else if (mine == 6) wave_product<6, NA, FWD>(d, U, w, acc, l);
+                else wave_product<NA, NA, FWD>(d, U, w, acc, l);
+            } else {
+                wave_product<NA, NA, FWD>(d, U, w, acc, l);
+            }
     }
     __syncthreads();
 #pragma unroll

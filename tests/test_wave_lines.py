@@ -56,6 +56,22 @@ def test_wave_inverse(gpu_ctx, ex, ey, N, per, bc):
         o.close()
 
 
+# the long kernels' output tiles per wave, two to seven: order 2 (no
+# antisymmetric parts) and the others, lines with and without a mirror symmetry
+@pytest.mark.gpu
+@pytest.mark.parametrize("ex,ey,N", [(129, 2, 2), (256, 2, 2), (160, 2, 4), (2, 200, 8), (256, 1, 7), (250, 3, 5)])
+@pytest.mark.parametrize("per,bc", ENDS)
+def test_long_wave_inverse(gpu_ctx, ex, ey, N, per, bc):
+    # bar and elements as in test_wave_inverse
+    m = se_amd.Mesh(gpu_ctx, (ex, ey), N, (0.0, 0.0), (float(ex), 1.25 * ey), per, bc)
+    h = se_amd.Helm(m, 1.0, 1.0, se_amd.DETJ_PHYSICAL)
+    r = np.random.default_rng(ex + N).standard_normal(m.n)
+    z = h.apply_fdm(r, se_amd.PREC_FP64)
+    assert np.linalg.norm(h.apply(z) - r) <= 1e-9 * np.linalg.norm(r)
+    h.close()
+    m.close()
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("order", [(0, 1), (1, 0)])
 def test_probe_of_a_batch_of_both_forms(gpu_ctx, order):
