@@ -105,10 +105,12 @@ __device__ __forceinline__ void wrap(const Line& l, double& c) {
     if (c > l.max) c = l.per ? l.min - l.max + c : l.max;
 }
 
-// The kernels take the order as a template argument NN (the launches
-// instantiate N = 2..8) or, with NN = 0, from the geometry (any N up to 12):
-// the same operations either way, with fixed trip counts and arrays of N + 1
-// when NN is known.
+// The kernels take the order as a template argument NN: the steps N = 2..12,
+// the others N = 2..8 and, with NN = 0, the order of the geometry: the same
+// operations either way, with fixed trip counts and arrays of N + 1 in registers
+// when NN is known.  (In scratch memory two lanes' arrays cost more than they
+// saved: 40 x 40 elements of order 9, first-order step, one lane 62 us, two 132,
+// two with the order known 30; 60 x 60 of order 12 330, 819, 152.)
 template <int NN> struct Ord {
     static constexpr int MAX = NN ? NN : 12;  // array bound
 };
@@ -202,9 +204,8 @@ struct Weights {
     // hides the weights from the compiler before a further sum, whose products
     // x y it would otherwise all keep from the one before
     __device__ __forceinline__ void fresh() {
-        if (NN)
 #pragma unroll
-            for (int j = 0; j <= NN; j++) asm volatile("" : "+v"(y[j]));
+        for (int j = 0; j <= NN; j++) asm volatile("" : "+v"(y[j]));
     }
 };
 template <int NN>
@@ -268,26 +269,19 @@ struct Rows {
         nd = nd_;
         dim = l.dim;
         pitch = g.nv0 * nd;
-        p = f + (size_t)node * nd + (NN && ND ? 0 : comp);
-        if (NN)
+        p = f + (size_t)node * nd + (ND ? 0 : comp);
 #pragma unroll
-            for (int jj = 0; jj < AHEAD && jj <= NN; jj++) read(jj);
+        for (int jj = 0; jj < AHEAD && jj <= NN; jj++) read(jj);
     }
-    __device__ __forceinline__ double sum(const SLGeom& g, const Weights<NN>& w) {
+    __device__ __forceinline__ double sum(const Weights<NN>& w) {
 #pragma clang fp contract(off)
         double s = 0.0;
-        if (NN) {
 #pragma unroll
-            for (int jj = 0; jj <= NN; jj++) {
+        for (int jj = 0; jj <= NN; jj++) {
 #pragma unroll
-                for (int ii = 0; ii <= NN; ii++) s += w.x[ii] * w.y[jj] * value(jj, ii);
-                asm volatile("" : "+v"(s) : : "memory");  // the next rows' reads stay behind this row's sum
-                if (jj + AHEAD <= NN) read(jj + AHEAD);
-            }
-        } else {
-            for (int jj = 0; jj <= g.N; jj++)
-                for (int ii = 0; ii <= g.N; ii++)
-                    s += w.x[ii] * w.y[jj] * p[(size_t)jj * pitch + (size_t)ii * nd];
+            for (int ii = 0; ii <= NN; ii++) s += w.x[ii] * w.y[jj] * value(jj, ii);
+            asm volatile("" : "+v"(s) : : "memory");  // the next rows' reads stay behind this row's sum
+            if (jj + AHEAD <= NN) read(jj + AHEAD);
         }
         return s;
     }
@@ -301,7 +295,7 @@ __device__ __forceinline__ double velocity_at(const SLGeom& g, const Line& l, do
     const Place p = place<NN>(l, c);
     Rows<NN, 2> r(g, l, p.node, vel, 2, l.dim);
     weights_at<NN>(g, p, w);
-    return r.sum(g, w);
+    return r.sum(w);
 }
 
 // Field::InterpGlobal at any point, one thread per point; vals node-major with
@@ -395,11 +389,11 @@ __device__ __forceinline__ void advected_at(const SLGeom& g, const Line& l, doub
     const Place p = place<NN>(l, c);
     Rows<NN, ND> r(g, l, p.node, q, nd, component(l, nd));
     weights_at<NN>(g, p, w);
-    a = r.sum(g, w);
+    a = r.sum(w);
     b = 0.0;
     if (ND == 0 && nd == 3) {
         w.fresh();
-        b = Rows<NN, 0>(g, l, p.node, q, nd, 2).sum(g, w);
+        b = Rows<NN, 0>(g, l, p.node, q, nd, 2).sum(w);
     }
 }
 // Stores node v's value, with Field::PeriodicUpdate (Field.cpp:232-252): the
@@ -464,12 +458,12 @@ __global__ void k_extrap(int n2, const double* __restrict__ vel, const double* _
 }
 
 // Advector::SecondOrder (Advector.cpp:203-246).  Four waves per SIMD (128
-// VGPRs, no spills; the bicubic form takes 256).  32x32 order 6 54 -> 19 us;
+// VGPRs, no spills; the bicubic form takes 256, orders above 8 130 to 166).  32x32 order 6 54 -> 19 us;
 // 96x96 order 6 135 -> 89 us: two thirds of it VALU issue (3300 instructions a
 // wave), the rest the cache's lookups of the gathers (126 us while a lane read 8
 // bytes at a time).
 template <int NN, int ND>
-__global__ __launch_bounds__(256, ND < 0 ? 2 : 4) void k_sl_second(SLGeom g, const double* __restrict__ q, const double* __restrict__ qp,
+__global__ __launch_bounds__(256, ND < 0 || NN > 8 ? 2 : 4) void k_sl_second(SLGeom g, const double* __restrict__ q, const double* __restrict__ qp,
                                                     int nd, const double* __restrict__ vel,
                                                     const double* __restrict__ vp1, const double* __restrict__ vph,
                                                     const double* __restrict__ vmh, double dt,
@@ -494,12 +488,12 @@ __global__ __launch_bounds__(256, ND < 0 ? 2 : 4) void k_sl_second(SLGeom g, con
         const Place p = place<NN>(l, c);
         Rows<NN, 2> rv(g, l, p.node, vel, 2, l.dim);
         weights_at<NN>(g, p, w);
-        h = c - 0.5 * dt * rv.sum(g, w);
+        h = c - 0.5 * dt * rv.sum(w);
         w.fresh();
-        a1 = Rows<NN, ND>(g, l, p.node, q, nd, component(l, nd)).sum(g, w);
+        a1 = Rows<NN, ND>(g, l, p.node, q, nd, component(l, nd)).sum(w);
         if (ND == 0 && nd == 3) {
             w.fresh();
-            b1 = Rows<NN, 0>(g, l, p.node, q, nd, 2).sum(g, w);
+            b1 = Rows<NN, 0>(g, l, p.node, q, nd, 2).sum(w);
         }
     }
     wrap(l, h);
@@ -670,7 +664,8 @@ int pair_blocks(int n) { return n / 128 + (n % 128 != 0); }  // two lanes per no
         default: hipLaunchKernelGGL(KERNEL<0>, GRID, dim3(256), 0, __VA_ARGS__); break; \
     }
 
-// KERNEL<N, the advected components: 1, 2, else 0; -1: bicubic>
+// KERNEL<N, the advected components: 1, 2, else 0; -1: bicubic> for the orders
+// 2..12 (se_sl_advect_dev, sl_second_check)
 #define SE_SL_ADV(KERNEL, N, GRID, ...)                                                                   \
     if (g.cubic) hipLaunchKernelGGL((KERNEL<N, -1>), GRID, dim3(256), 0, __VA_ARGS__);                   \
     else if (nd == 1) hipLaunchKernelGGL((KERNEL<N, 1>), GRID, dim3(256), 0, __VA_ARGS__);               \
@@ -685,7 +680,10 @@ int pair_blocks(int n) { return n / 128 + (n % 128 != 0); }  // two lanes per no
         case 6: SE_SL_ADV(KERNEL, 6, GRID, __VA_ARGS__); break;       \
         case 7: SE_SL_ADV(KERNEL, 7, GRID, __VA_ARGS__); break;       \
         case 8: SE_SL_ADV(KERNEL, 8, GRID, __VA_ARGS__); break;       \
-        default: SE_SL_ADV(KERNEL, 0, GRID, __VA_ARGS__); break;      \
+        case 9: SE_SL_ADV(KERNEL, 9, GRID, __VA_ARGS__); break;       \
+        case 10: SE_SL_ADV(KERNEL, 10, GRID, __VA_ARGS__); break;     \
+        case 11: SE_SL_ADV(KERNEL, 11, GRID, __VA_ARGS__); break;     \
+        default: SE_SL_ADV(KERNEL, 12, GRID, __VA_ARGS__); break;     \
     }
 
 struct SLScratch {
