@@ -357,24 +357,16 @@ __device__ __forceinline__ int opaque_tid() {
     return tid;
 }
 
-// Batched: work items (member, tile); MODE's partials go to the member's
-// `part` (line_tiles of its mesh entries).
-// gated: a member whose `gate` CG is not awaiting its true-residual check
-// (the direction kernel before this launch marks it) has nothing to do.
+// Batched, members of one order: work items (member, tile), a workgroup each.
 // Four workgroups per CU (at most 128 VGPRs; at N = 8 a few values spill to
-// scratch): 4% faster on the ensemble than three at 145 VGPRs.
-template <int N, int MODE>
+// scratch): LDS then sets the occupancy, not the registers.
+template <int N>
 __global__ __launch_bounds__(256, 4) void k_apply_lines_batch(const ApplyMember* __restrict__ members,
-                                                            const int2* __restrict__ work, int nwork, int gated) {
+                                                            const int2* __restrict__ work) {
     SE_LINE_LDS(N, lds);
-    for (int w = blockIdx.x; w < nwork; w += gridDim.x) {
-        const int2 it = work[w];
-        if (it.x < 0) continue;  // a padding item of an XCD-ordered list
-        const ApplyMember& a = members[it.x];
-        if (gated && a.gate && a.gate->status != CG_PENDING) continue;
-        __syncthreads();  // the previous item's LDS reads are done
-        apply_lines_tile<N, MODE>(lds, opaque_tid(), a.P, it.y, a.in, a.out, a.part, a.np, a.b);
-    }
+    const int2 it = work[blockIdx.x];
+    const ApplyMember& a = members[it.x];
+    apply_lines_tile<N, AP_PLAIN>(lds, threadIdx.x, a.P, it.y, a.in, a.out, nullptr, 0);
 }
 
 // The same over members of any orders at once: the orders' tiles run side by
@@ -382,6 +374,9 @@ __global__ __launch_bounds__(256, 4) void k_apply_lines_batch(const ApplyMember*
 // each at small sizes (24 channel states of six orders: 78 -> 19 us; the
 // 512-member ensemble, three orders of many tiles each, is unchanged).  One
 // LDS pool, the largest order's: N = 8 holds four workgroups a CU either way.
+// MODE's partials go to the member's `part` (line_tiles of its mesh entries).
+// gated: a member whose `gate` CG is not awaiting its true-residual check
+// (the direction kernel before this launch marks it) has nothing to do.
 template <int MODE>
 __global__ __launch_bounds__(256, 4) void k_apply_lines_any(const ApplyMember* __restrict__ members,
                                                           const int2* __restrict__ work, int nwork, int gated) {

@@ -14,7 +14,9 @@
 // v_mfma_f32_32x32x16_bf16 (BF16 operands, FP32 accumulation).  Matrices are
 // padded to multiples of 64 with zeros; pass 1 reads the FP64 residual with
 // its true extent and pass 4 writes the FP64 result with it, together with
-// per-tile partial sums of r.z, sum z and sum r.
+// per-tile partial sums of r.z, sum z and sum r.  Lines of up to 256 elements
+// take the plane-wave form instead (wave_host.h, fdm_wave.h), in every precision
+// but BF16 operands throughout (fdm_wave below).
 //
 // The solver around it is FP64 CG (x0 = 0, true-residual stop, constant null
 // space by Euclidean-mean projection, as the Jacobi-PCG of helm.hip) whose
@@ -24,7 +26,7 @@
 // launch per phase over (member, item) work lists, one host pull of the
 // members' states per round; a single solve is a batch of one, so batched
 // results are the single ones bit for bit.  The exact FP64 operator apply is
-// k_apply_lines_batch; every reduction is per item with consumer-side
+// k_apply_lines_any; every reduction is per item with consumer-side
 // fixed-order sums.
 #include <hip/hip_bf16.h>
 #include <hip/hip_runtime.h>
@@ -904,6 +906,7 @@ int wave_line_of(const se_op* op, int axis, std::shared_ptr<const WaveLineDev>& 
     if (!rc) rc = up(w->tiles, tf.data(), sizeof(WaveTile) * tf.size());
     if (!rc) rc = up(w->phi, L.phi.data(), sizeof(double) * L.phi.size());
     if (rc) return rc;
+    for (auto& f : w->L.F) std::vector<double>().swap(f);  // (the device has them in operand order)
     g_wave_cache[key] = w;
     out = w;
     return SE_OK;
@@ -1087,7 +1090,6 @@ WaveTask wave_task(const se_op* op, const double* r, double* z, double* part, in
     t.y = dim(*F->wy);
     t.N = F->wx->L.N;
     t.nS = F->wx->L.nS;
-    t.nA = F->wx->L.nA;
     t.t1 = F->wt1.as<double>();
     t.r = r;
     t.z = z;

@@ -53,7 +53,7 @@ struct WaveDim {
 };
 struct WaveTask {
     WaveDim x, y;
-    int N, nS, nA;
+    int N, nS;
     double* t1;                       // [y blocks of 1 << x.logR][x modes][1 << x.logR]
     const double *r, *b;              // the residual; the right-hand side (first direction)
     double *z, *p;                    // result; the CG's direction
