@@ -698,16 +698,26 @@ struct GridStay {
 
 // The solve as one launch.  done = false: not of this form (too large for the
 // chip's LDS and registers, an SVV term, a recorded history), or a wait ran
-// out, now or in solves before it; f is whole then (d_x may
-// hold part of a result: workgroups past the last sum have stored theirs) and
-// the caller solves it launch by launch.
+// out, now or in solves before it; f is whole then (d_x may hold part of a
+// result: workgroups past the last sum have stored theirs) and the caller
+// solves it launch by launch.
 int pcg_grid(se_op* op, const double* d_f, double* d_x, const se_solve_opts& o, se_solve_info& info, bool& done) {
     done = false;
     se_mesh* m = op->mesh;
     se_ctx* c = m->ctx;
     if (o.history || op->svv_mN > 0 || m->n < 1 || c->device >= kDevices) return SE_OK;
+    // the tile depends on the mesh and the device only: chosen once per operator
+    int(&tile)[3] = op->grid_tile;
     GridShape sh;
-    if (!grid_shape(m, c->cu_count, sh)) return SE_OK;
+    if (tile[2] == 0) {
+        const bool fits = grid_shape(m, c->cu_count, sh);
+        tile[0] = sh.tx, tile[1] = sh.ty, tile[2] = fits ? sh.T : -1;
+    } else if (tile[2] > 0) {
+        sh.tx = tile[0], sh.ty = tile[1], sh.T = tile[2];
+        sh.G = ((m->nEls[0] + sh.tx - 1) / sh.tx) * ((m->nEls[1] + sh.ty - 1) / sh.ty);
+        sh.lds = grid_lds(m->N, sh.tx, sh.ty, sh.T, sh.G);
+    }
+    if (tile[2] < 0) return SE_OK;
     GridGate& gate = g_gate[c->device];
     if (sh.G > 1 && gate.leaves_out()) return SE_OK;
     hipStream_t s = c->stream;

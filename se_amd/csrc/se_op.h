@@ -36,6 +36,7 @@ struct se_op {
     se::DevBuf grid_slots, grid_work;        // one-launch solve (pcg_grid.hip): sum slots, work
     bool grid_dirty = false;                 // they need clearing first
     int grid_turn = 0;                       // the region the next solve uses
+    int grid_tile[3] = {0, 0, 0};            // its tile's elements and threads (0: not chosen, -1: none fits)
     hipGraphExec_t graph_exec_lo = nullptr;
     int graph_iters_lo = 0;
     // spectral vanishing viscosity term (svv.hip): dt, cutoff (0: none), the
