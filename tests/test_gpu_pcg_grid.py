@@ -12,12 +12,16 @@ pytestmark = pytest.mark.gpu
 
 PER, XPER, NONE = (1, 1), (1, 0), (0, 0)
 # one tile with its own seams, one per direction, ragged last tiles, many small
-# tiles, every boundary kind, orders 2..8 and the wide-tile form
+# tiles, every boundary kind, orders 2..8, and tiles of 576 threads: one alone
+# (orders 3, 4), and several with walls and ragged last ones, with the diagonal
+# in registers (order 6) and read from memory (orders 7, 8)
 CASES = [
     ((1, 1), 4, PER, (0, 0, 0, 0)), ((8, 8), 4, PER, (0, 0, 0, 0)), ((3, 40), 3, PER, (0, 0, 0, 0)),
     ((40, 3), 3, XPER, (1, 1, 0, 0)), ((23, 17), 2, NONE, (1, 1, 1, 1)), ((19, 21), 5, NONE, (1, 0, 0, 0)),
     ((31, 29), 6, XPER, (1, 1, 0, 0)), ((17, 13), 7, NONE, (0, 1, 1, 0)), ((50, 61), 8, PER, (0, 0, 0, 0)),
     ((80, 70), 6, NONE, (1, 1, 1, 1)),
+    ((130, 101), 6, XPER, (1, 1, 0, 0)), ((100, 91), 7, NONE, (1, 1, 1, 1)), ((110, 90), 7, XPER, (0, 1, 0, 0)),
+    ((120, 115), 8, NONE, (0, 1, 1, 0)), ((96, 96), 8, PER, (0, 0, 0, 0)),
 ]
 
 
@@ -28,6 +32,7 @@ def test_grid_solve(gpu_ctx, nEls, N, per, bc):
     h = se_amd.Helm(m, 40.0, 1.0, se_amd.DETJ_PHYSICAL)
     rng = np.random.default_rng(N)
     f = rng.standard_normal(m.n)
+    launches = gpu_ctx.solver_counts()[0]
     # the same iterates: a few iterations, whose round-off grows by less than 100 eps each
     for k in (1, 6):
         x, i = h.pcg(f, maxit=k)
@@ -47,6 +52,7 @@ def test_grid_solve(gpu_ctx, nEls, N, per, bc):
     f[m.n // 2] = np.nan
     _, j = h.pcg(f)
     assert j["status"] == se_amd.SOLVE_NONFINITE
+    assert gpu_ctx.solver_counts()[0] == launches + 5  # every solve without a history was one launch
     h.close()
     m.close()
 
@@ -55,7 +61,9 @@ def test_grid_null_space(gpu_ctx):
     m = se_amd.Mesh(gpu_ctx, (21, 18), 5, (0.0, 0.0), (1.0, 1.0), PER, (0, 0, 0, 0))
     h = se_amd.Helm(m, 0.0, -1.0, se_amd.DETJ_LITERAL)
     f = np.random.default_rng(1).standard_normal(m.n)
+    launches = gpu_ctx.solver_counts()[0]
     x, i = h.pcg(f, null_space=True)
+    assert gpu_ctx.solver_counts()[0] == launches + 1
     y, _ = h.pcg(f, null_space=True, history=True, maxit=5000)
     assert i["status"] == 0
     r = (f - f.mean()) - h.apply(x)
@@ -71,13 +79,40 @@ def test_grid_wait_runs_out(gpu_ctx):
     h = se_amd.Helm(m, -50.0, -1.0, se_amd.DETJ_LITERAL)
     f = np.random.default_rng(2).standard_normal(m.n)
     y, j = h.pcg(f, history=True, maxit=5000)
+    launches, gave_up = gpu_ctx.solver_counts()
     os.environ["SE_GRID_WAIT"] = "0"
     try:
         x, i = h.pcg(f)
     finally:
         del os.environ["SE_GRID_WAIT"]
+    assert gpu_ctx.solver_counts() == (launches, gave_up + 1)
     assert i["status"] == 0 and i["iters"] == j["iters"] and np.array_equal(x, y)
     x, i = h.pcg(f)  # and the next solve is whole again
+    assert gpu_ctx.solver_counts() == (launches + 1, gave_up + 1)
     assert i["status"] == 0 and np.linalg.norm(f - h.apply(x)) <= 1.01e-10 * np.linalg.norm(f)
+    h.close()
+    m.close()
+
+
+@pytest.mark.parametrize("nEls,N", [((24, 24), 6), ((96, 96), 8)])
+def test_grid_restarts_from_the_true_residual(gpu_ctx, nEls, N):
+    """A target below what b - A x can reach: the recursion meets it (the other
+    solver's history shows where), the check fails, and the solve goes on from
+    the true residual to the iteration limit with a whole x."""
+    m = se_amd.Mesh(gpu_ctx, nEls, N, (0.0, 0.0), (1.0, 1.0), XPER, (1, 1, 0, 0))
+    h = se_amd.Helm(m, 4e3, 1.0, se_amd.DETJ_PHYSICAL)
+    f = np.random.default_rng(7).standard_normal(m.n)
+    _, i = h.pcg(f, rtol=1e-12)
+    assert i["status"] == 0
+    limit = 2 * i["iters"]
+    _, j = h.pcg(f, rtol=1e-16, maxit=limit, history=True)
+    met = int(np.argmax(j["hist"] <= 1e-16))
+    assert 0 < met < limit - 20 and j["status"] == se_amd.SOLVE_MAXIT
+    launches = gpu_ctx.solver_counts()[0]
+    x, i = h.pcg(f, rtol=1e-16, maxit=limit)
+    assert gpu_ctx.solver_counts()[0] == launches + 1
+    assert i["status"] == se_amd.SOLVE_MAXIT and i["iters"] == limit
+    assert 1e-16 < i["true_rel_residual"] <= 1e-12
+    assert np.linalg.norm(f - h.apply(x)) <= 1.01e-12 * np.linalg.norm(f)
     h.close()
     m.close()
