@@ -96,13 +96,28 @@ SE_POW_FN double log_hi_lo(uint64_t ix, double* tail) {
     return y;
 }
 
-// exp(x + xtail) with the sign of the result in sign_bias
-SE_POW_FN double exp_hi_lo(double x, double xtail, uint64_t sign_bias) {
+// exp(x + xtail) = 2^(ki / 128) (1 + tmp): the bits of the scale (exponent
+// perhaps out of range) are returned
+SE_POW_FN uint64_t exp_parts(double x, double xtail, uint64_t& ki, double& tmp) {
 #pragma clang fp contract(off)
     const double InvLn2N = 0x1.71547652b82fep0 * 128, Shift = 0x1.8p52, NegLn2hiN = -0x1.62e42fefa0000p-8,
                  NegLn2loN = -0x1.cf79abc9e3b3ap-47;
     const double C2 = 0x1.ffffffffffdbdp-2, C3 = 0x1.555555555543cp-3, C4 = 0x1.55555cf172b91p-5,
                  C5 = 0x1.1111167a4d017p-7;
+    double kd = fma(InvLn2N, x, Shift);
+    ki = bits(kd);
+    kd -= Shift;
+    double r = fma(kd, NegLn2loN, fma(kd, NegLn2hiN, x));
+    r += xtail;
+    const uint64_t idx = 2 * (ki % 128);
+    const double tail = from_bits(kPowExpTab[idx]), r2 = r * r;
+    tmp = fma(r2 * r2, fma(r, C5, C4), fma(r2, fma(r, C3, C2), tail + r));
+    return kPowExpTab[idx + 1] + (ki << 45);
+}
+
+// exp(x + xtail) with the sign of the result in sign_bias
+SE_POW_FN double exp_hi_lo(double x, double xtail, uint64_t sign_bias) {
+#pragma clang fp contract(off)
     uint32_t abstop = (uint32_t)(bits(x) >> 52) & 0x7ff;
     if (abstop - 0x3c9u >= 0x408u - 0x3c9u) {  // |x| < 2^-54 or |x| >= 512
         if (abstop - 0x3c9u >= 0x80000000u) {
@@ -115,17 +130,9 @@ SE_POW_FN double exp_hi_lo(double x, double xtail, uint64_t sign_bias) {
         }
         abstop = 0;
     }
-    double kd = fma(InvLn2N, x, Shift);
-    const uint64_t ki = bits(kd);
-    kd -= Shift;
-    double r = fma(kd, NegLn2loN, fma(kd, NegLn2hiN, x));
-    r += xtail;
-    const uint64_t idx = 2 * (ki % 128);
-    const uint64_t top = (ki + sign_bias) << 45;
-    const double tail = from_bits(kPowExpTab[idx]);
-    uint64_t sbits = kPowExpTab[idx + 1] + top;
-    const double r2 = r * r;
-    const double tmp = fma(r2 * r2, fma(r, C5, C4), fma(r2, fma(r, C3, C2), tail + r));
+    uint64_t ki;
+    double tmp;
+    uint64_t sbits = exp_parts(x, xtail, ki, tmp) + (sign_bias << 45);
     if (abstop == 0) {
         // scale's exponent may be out of range: glibc's specialcase (no FMAs)
         if ((ki & 0x80000000ULL) == 0) {
@@ -213,25 +220,13 @@ SE_POW_FN double pow_plain_at(double x, double hi, double lo, int k) {
 #pragma clang fp contract(off)
     if (k == 0) return 1.0;
     if (k == 1) return x;
-    const double InvLn2N = 0x1.71547652b82fep0 * 128, Shift = 0x1.8p52, NegLn2hiN = -0x1.62e42fefa0000p-8,
-                 NegLn2loN = -0x1.cf79abc9e3b3ap-47;
-    const double C2 = 0x1.ffffffffffdbdp-2, C3 = 0x1.555555555543cp-3, C4 = 0x1.55555cf172b91p-5,
-                 C5 = 0x1.1111167a4d017p-7;
     const double y = (double)k;
     const double ehi = y * hi;
     const double elo = fma(y, lo, fma(y, hi, -ehi));
-    double kd = fma(InvLn2N, ehi, Shift);
-    const uint64_t ki = bits(kd);
-    kd -= Shift;
-    double r = fma(kd, NegLn2loN, fma(kd, NegLn2hiN, ehi));
-    r += elo;
-    const uint64_t idx = 2 * (ki % 128);
+    uint64_t ki;
+    double tmp;
     // an odd power carries x's sign
-    const uint64_t top = (ki << 45) + ((k & 1) ? bits(x) & 0x8000000000000000ULL : 0);
-    const double tail = from_bits(kPowExpTab[idx]);
-    const uint64_t sbits = kPowExpTab[idx + 1] + top;
-    const double r2 = r * r;
-    const double tmp = fma(r2 * r2, fma(r, C5, C4), fma(r2, fma(r, C3, C2), tail + r));
+    const uint64_t sbits = exp_parts(ehi, elo, ki, tmp) + ((k & 1) ? bits(x) & 0x8000000000000000ULL : 0);
     const double scale = from_bits(sbits);
     return fma(scale, tmp, scale);
 }
