@@ -8,15 +8,17 @@ Workloads (--workload):
       right-hand sides f = M g with g a seeded random field with an isotropic
       k^-3 spectrum.  One step = all 512 solves to a true relative residual of
       1e-10, batched: FP64 CG preconditioned by fast diagonalisation with its
-      transforms on the matrix cores (--precision fp64_bf16c, the default:
-      FP64 transforms for the first application, BF16 operands for the
-      corrections; fp64_fp32c: FP32 corrections; fp64, fp32_ir, bf16_ir:
-      FP64, FP32 or BF16 operands throughout;
+      transforms on the matrix cores.  --precision names the least precision a
+      solve asks for (fp64_bf16c, the default: FP64 for the first application,
+      BF16 operands for the corrections; fp64_fp32c: FP32 corrections; fp64,
+      fp32_ir, bf16_ir: FP64, FP32 or BF16 operands throughout): on lines of up
+      to 256 elements, as all of these, every choice but bf16_ir runs the same
+      FP64 plane-wave transforms, and the line's dtype says so.
       --pc jacobi: the reference's Jacobi-PCG with FP32 or BF16 inner
-      iterations and FP64 reliable updates).  The plain FP64 GPU path
+      iterations and FP64 reliable updates.  The plain FP64 GPU path
       (each member alone, FP64 Jacobi-PCG, the reference's algorithm) is timed
       on the same members once and reported beside it, with the other
-      precisions / preconditioners batched, and a served two-layer QG stream of
+      transforms / preconditioners batched, and a served two-layer QG stream of
       16 requests for the metric's p50/p99 latency.
   helmholtz_128 -- one solve on 128x128 elements at p = 8 (1 048 576
       unknowns), lambda = 100, same kind of right-hand side.
@@ -49,8 +51,22 @@ FP64_PEAK_TFLOPS = 78.6        # MI355X FP64 vector
 MFMA_PEAK_TFLOPS = {"fp64": 78.6, "fp64_fp32c": 78.6, "fp64_bf16c": 78.6, "fp32_ir": 157.3, "bf16_ir": 2500.0}
 DTYPE = {"fp64": "f64", "fp64_fp32c": "f64+f32", "fp64_bf16c": "f64+bf16", "fp32_ir": "f32+f64",
          "bf16_ir": "bf16+f64"}
+# periodic and walled lines of this many elements at most have plane-wave FDM
+# transforms: FP64 in every precision but bf16_ir
+WAVE_ELEMENTS = 256
 # the element type of the probed GEMM (for fp64_*c: the first application's, FP64)
 GEMM_T = {"fp64": "double", "fp64_fp32c": "double", "fp64_bf16c": "double", "fp32_ir": "float", "bf16_ir": "bf16"}
+
+
+def waves(prec_name, pc, cfgs):
+    """The FDM transforms of all these problems run as FP64 plane waves."""
+    import se_amd
+    return pc == se_amd.PC_FDM and prec_name != "bf16_ir" and all(max(c["nEls"]) <= WAVE_ELEMENTS for c in cfgs)
+
+
+def dtype_of(prec_name, pc, cfgs):
+    """The types a line's solves compute in."""
+    return "f64" if waves(prec_name, pc, cfgs) else DTYPE[prec_name]
 
 
 def prec_code(name):
@@ -66,9 +82,9 @@ def parse():
     p.add_argument("--warmup", type=int, default=2)
     p.add_argument("--workload", default="ensemble_512")
     p.add_argument("--precision", default=None, choices=["fp64", "fp64_fp32c", "fp64_bf16c", "fp32_ir", "bf16_ir"],
-                   help="default: fp64_bf16c (FDM: first application on the FP64 matrix cores, corrections "
-                        "with BF16 operands) for ensemble_512, fp32_ir for "
-                        "qg2_stream, fp64 for helmholtz_*")
+                   help="the least precision: default fp64_bf16c (FDM: first application in FP64, corrections "
+                        "with BF16 operands; on lines of up to 256 elements FP64 throughout) for ensemble_512, "
+                        "fp32_ir for qg2_stream, fp64 for helmholtz_*")
     p.add_argument("--pc", default="default", choices=["default", "jacobi", "fdm"],
                    help="preconditioner: default = FDM for ensemble_512 and the mixed precisions, Jacobi (the "
                         "reference's algorithm) for fp64 on helmholtz_* and qg2_stream")
@@ -217,15 +233,14 @@ def pc_code(a, prec_name, fdm_default=False):
     return se_amd.PC_JACOBI
 
 
-def fdm_roofline(pr, prec_name):
+def fdm_roofline(pr, prec_name, wave):
     """pr: us / flops of the FDM's four 1-D transforms and us / bytes of the FP64
-    apply.  BF16 transforms are four launches of the dense GEMM, bound by the
-    matrix cores.  The others run as plane waves over the elements in FP64, in
-    three launches -- x, both transforms of y (half of its time in each of two
-    entries), and back in x -- each of which reads and writes the unknowns once."""
+    apply.  Dense transforms are four launches of the GEMM, bound by the matrix
+    cores.  Plane waves over the elements (FP64) are three launches -- x, both
+    transforms of y (half of its time in each of two entries), and back in x --
+    each of which reads and writes the unknowns once."""
     apply_gbs = pr["bytes_apply"] / (pr["us_apply"] * 1e-6) / 1e9
     ps = list(zip(pr["us_pass"], pr["flops_pass"]))
-    wave = prec_name != "bf16_ir"
     if wave:
         ps = [ps[0], (ps[1][0] + ps[2][0], ps[1][1] + ps[2][1]), ps[3]]
     us, fl = sum(u for u, _ in ps), sum(f for _, f in ps)
@@ -287,7 +302,7 @@ def run_ensemble(a, prec_name):
     if pc == se_amd.PC_FDM:
         # dominant kernel: the FDM transforms on the matrix cores (each launch
         # over all members, timed back to back after the last solve)
-        roof = fdm_roofline(b.fdm_probe(reps=a.probe_reps), prec_name)
+        roof = fdm_roofline(b.fdm_probe(reps=a.probe_reps), prec_name, waves(prec_name, pc, cfgs))
         roof["traffic"] = pmc_traffic(roof, "%s__ensemble_512_%s_pmc.md" % (roof["kernel"].split("<")[0],
                                                                             prec_name.split("_")[0]))
     else:
@@ -320,17 +335,16 @@ def run_ensemble(a, prec_name):
         config.update({"fp64_gpu_value": v64, "fp64_gpu_ms": ms64, "speedup_vs_fp64_gpu": value / v64,
                        "fp64_all_converged": all(i["status"] == 0 for i in res64[-1]),
                        "max_rel_diff_vs_fp64_solution": diff})
-        # the other legs of the same batch, to separate the gains: batching
-        # (FP64 FDM batched), precision (this line's FDM at another
-        # precision) and the preconditioner (the inner Jacobi-PCG mixed solve)
+        # the other legs of the same batch, to separate the gains: the
+        # transforms (FP64 plane waves, BF16 operands) and the preconditioner
+        # (the inner Jacobi-PCG mixed solve).  On lines of up to 256 elements
+        # the other FDM precisions are the FP64 leg's computation.
         legs = {}
-        for lab, p2, c2 in (("fp64_fdm_batched", se_amd.PREC_FP64, se_amd.PC_FDM),
-                            ("fp64_fp32c_fdm_batched", se_amd.PREC_FP64_FP32C, se_amd.PC_FDM),
-                            ("fp64_bf16c_fdm_batched", se_amd.PREC_FP64_BF16C, se_amd.PC_FDM),
-                            ("fp32_fdm_batched", se_amd.PREC_FP32_IR, se_amd.PC_FDM),
-                            ("bf16_fdm_batched", se_amd.PREC_BF16_IR, se_amd.PC_FDM),
-                            ("fp32_jacobi_batched", se_amd.PREC_FP32_IR, se_amd.PC_JACOBI)):
-            if p2 == prec and c2 == pc:
+        for lab, name, c2 in (("fp64_fdm_batched", "fp64", se_amd.PC_FDM),
+                              ("bf16_fdm_batched", "bf16_ir", se_amd.PC_FDM),
+                              ("fp32_jacobi_batched", "fp32_ir", se_amd.PC_JACOBI)):
+            p2 = prec_code(name)
+            if (p2 == prec and c2 == pc) or (waves(name, c2, cfgs) and waves(prec_name, pc, cfgs)):
                 continue
             xs2 = [torch.zeros_like(x) for x in xs]
             xp2 = [x.data_ptr() for x in xs2]
@@ -358,7 +372,7 @@ def run_ensemble(a, prec_name):
     if not a.no_cpu_baseline:
         iters_ref = [i["iters"] for i in res64[-1]] if not a.no_fp64 else [i["iters"] for i in infos]
         cpu = ensemble_cpu(a, cfgs, hs, fs, iters_ref)
-    return base_line(a, value, ms, DTYPE[prec_name], config, roof, cpu)
+    return base_line(a, value, ms, dtype_of(prec_name, pc, cfgs), config, roof, cpu)
 
 
 def ensemble_cpu(a, cfgs, hs, fs, iters_ref):
@@ -428,7 +442,7 @@ def run_single(a, prec_name):
               "all_converged": ok, "n_iter_per_s": m.n * info["iters"] / (ms * 1e-3), "wall_s_timed": t_wall}
     T = GEMM_T[prec_name]
     if pc == se_amd.PC_FDM:
-        roof = fdm_roofline(h.fdm_probe(reps=a.probe_reps), prec_name)
+        roof = fdm_roofline(h.fdm_probe(reps=a.probe_reps), prec_name, waves(prec_name, pc, [cfg]))
     elif prec == se_amd.PREC_FP64:
         # dominant kernel: the FP64 operator apply, timed on its stream
         for _ in range(5):
@@ -460,11 +474,13 @@ def run_single(a, prec_name):
                        "max_rel_diff_vs_fp64_solution":
                            float(torch.linalg.norm(d_x - d_x64) / torch.linalg.norm(d_x64))})
         legs = {}
-        for lab, p2, c2 in (("fp64_fdm", se_amd.PREC_FP64, se_amd.PC_FDM),
-                            ("fp32_fdm", se_amd.PREC_FP32_IR, se_amd.PC_FDM),
-                            ("bf16_fdm", se_amd.PREC_BF16_IR, se_amd.PC_FDM),
-                            ("fp32_jacobi", se_amd.PREC_FP32_IR, se_amd.PC_JACOBI)):
-            if p2 == prec and c2 == pc:
+        for lab, name, c2 in (("fp64_fdm", "fp64", se_amd.PC_FDM),
+                              ("fp32_fdm", "fp32_ir", se_amd.PC_FDM),
+                              ("bf16_fdm", "bf16_ir", se_amd.PC_FDM),
+                              ("fp32_jacobi", "fp32_ir", se_amd.PC_JACOBI)):
+            p2 = prec_code(name)
+            # (FP32 FDM is the FP64 leg's computation where both are plane waves)
+            if (p2 == prec and c2 == pc) or (waves(name, c2, [cfg]) and (lab == "fp32_fdm" or waves(prec_name, pc, [cfg]))):
                 continue
             d_x2 = torch.empty_like(d_x)
             solve(p2, d_x2, c2)
@@ -487,7 +503,7 @@ def run_single(a, prec_name):
                          "system, %d threads (and 1), scaled to the reference algorithm's %d-iteration solve; "
                          "CSR assembly %.1f s not counted" % (s["iters"], s["nnz"], nth, it_ref, s["t_asm"]),
                "seconds_per_iteration": s["t_it"], "seconds_per_iteration_1_thread": s1["t_it"]}
-    return base_line(a, value, ms, DTYPE[prec_name], config, roof, cpu)
+    return base_line(a, value, ms, dtype_of(prec_name, pc, [cfg]), config, roof, cpu)
 
 
 def stream_requests(n):
@@ -571,7 +587,7 @@ def run_stream(a, prec_name):
                        "fp64_latency_p50_s": stream_summary(r64)["latency_p50_s"],
                        "fp64_latency_p99_s": stream_summary(r64)["latency_p99_s"],
                        "speedup_vs_fp64_gpu": r64["wall"] / r["wall"]})
-    return base_line(a, value, r["wall"] * 1e3, DTYPE[prec_name], config, None, None)
+    return base_line(a, value, r["wall"] * 1e3, dtype_of(prec_name, pc, reqs), config, None, None)
 
 
 def main():
