@@ -54,16 +54,19 @@ enum { SE_DETJ_LITERAL = 0, SE_DETJ_PHYSICAL = 1 };
  * the one that sets the residual's floor -- runs in FP64 and later ones,
  * corrections of the residual it left, may run in FP32, resp. with BF16
  * operands.  These are the least precisions: FDM transforms of lines of up to
- * 256 elements run in FP64 in every one of them but BF16_IR (their plane-wave
- * form is faster there than dense transforms of fewer bits). */
+ * 256 elements (255 between two natural ends) run in FP64 in every one of them
+ * but BF16_IR (their plane-wave form is faster there than dense transforms of
+ * fewer bits).  A solve stops at the first iterate whose true residual meets
+ * rtol, whatever the precision: with FP64 transforms that is often the first,
+ * just below rtol, where dense FP32 ones overshot it in a second or third. */
 enum { SE_PREC_FP64 = 0, SE_PREC_FP32_IR = 1, SE_PREC_BF16_IR = 2, SE_PREC_FP64_FP32C = 3, SE_PREC_FP64_BF16C = 4 };
 
 /* Preconditioner.  JACOBI: the reference's (PETSc -pc_type jacobi; FP64) or
  * the inner Jacobi-PCG with FP64 reliable updates (FP32_IR / BF16_IR).
- * FDM: fast diagonalisation of the operator's separable form (dense 1-D
- * eigenvector transforms on the matrix cores, in the solve's precision)
- * inside FP64 CG -- a near-exact inverse on the reference's uniform meshes,
- * so the CG needs a handful of iterations.  DEFAULT: JACOBI for FP64, FDM for
+ * FDM: fast diagonalisation of the operator's separable form (plane waves over
+ * the elements of a line, or dense 1-D eigenvector transforms, on the matrix
+ * cores) inside FP64 CG -- a near-exact inverse on the reference's uniform
+ * meshes, so the CG needs a handful of iterations.  DEFAULT: JACOBI for FP64, FDM for
  * FP32_IR / BF16_IR. */
 enum { SE_PC_DEFAULT = 0, SE_PC_JACOBI = 1, SE_PC_FDM = 2 };
 
@@ -181,14 +184,16 @@ typedef struct {
     int maxit;          /* iteration limit, inner iterations counted (default 100000) */
     int precision;      /* SE_PREC_* (default FP64) */
     int null_space;     /* 1: constant null space (periodic Poisson) */
-    int check_every;    /* iterations per graph replay (default 32).  FP64: a host convergence
-                           check after every replay.  Mixed precision (single and batched):
+    int check_every;    /* iterations per graph replay (default 32).  FP64 launch by launch: a host
+                           convergence check after every replay (a solve in one launch checks
+                           every iteration on the device).  Mixed precision (single and batched):
                            after every replay for the first 16 checks, then after every 2nd,
                            from the 32nd check on after every 4th */
     double inner_rtol;  /* mixed solves: reliable update once the recursive residual
                            fell by this factor since the last one (0 = 0.1) */
     int max_outer;      /* limit on FP64 reliable updates of a mixed solve (default 1000) */
-    double* history;    /* optional host array, maxit+1 recursive relative residuals (FP64 only) */
+    double* history;    /* optional host array, maxit+1 recursive relative residuals (FP64 only);
+                           the solve then runs launch by launch (see se_helm_pcg) */
     int preconditioner; /* SE_PC_* (default SE_PC_DEFAULT) */
 } se_solve_opts;
 
@@ -235,7 +240,17 @@ int se_helm_probe(se_op* op, int precision, int reps, double* us_dir, double* us
                   double* bytes_upd);
 /* Jacobi-PCG on A x = f, x0 = 0  [ref: KSPSolve with -ksp_type cg -pc_type
  *  jacobi, src/linsys/HelmholtzEqn.cpp:120-131] (sign-normalised: a
- *  negative-definite A is solved as -A x = -f) */
+ *  negative-definite A is solved as -A x = -f)
+ * An FP64 Jacobi-PCG whose element tiles all fit the device at once (order 8:
+ * 128 x 128 elements on 256 CUs; more at lower orders) runs as one launch; larger
+ * systems, operators with an SVV term and solves with a history run launch by
+ * launch.  The two add in different orders: the same recurrence and stopping
+ * test, results that differ by round-off, so a recorded history is that of the
+ * solve with it.  Which one runs depends on the call alone -- solves from several
+ * threads of a process wait for each other's CUs -- unless the device is so
+ * taken up by another process that workgroups of a launch are not resident
+ * together within 0.1 s: that solve is repeated launch by launch
+ * (se_ctx_solver_counts). */
 int se_helm_pcg_dev(se_op* op, const double* d_f, double* d_x, const se_solve_opts* opts, se_solve_info* info);
 int se_helm_pcg(se_op* op, const double* f, double* x, const se_solve_opts* opts, se_solve_info* info);
 /* full HelmholtzEqn::Solve: f = M rhs + b, solve, UpdateField into sol_field

@@ -815,8 +815,8 @@ std::mutex g_wave_mu;
 std::map<std::string, std::weak_ptr<const WaveLineDev>> g_wave_cache;
 
 // axis of op's mesh: the wave form of its line; null if the line has none.
-// The element tables are the mean over the elements (equal up to round-off on
-// the uniform mesh).
+// The element tables are the mean over the elements (on the uniform mesh they
+// drift by ~1e-11 at order 8, wave_host.h).
 int wave_line_of(const se_op* op, int axis, std::shared_ptr<const WaveLineDev>& out) {
     const se_mesh* m = op->mesh;
     const int N = m->N, n1 = N + 1, CS = 4 * n1 + n1 * n1, ne = m->nEls[axis], per = m->periodic[axis];
@@ -1044,11 +1044,20 @@ int wave_modes_prepare(se_op* op, FdmOp* F) {
 
 // op's transforms in this precision take the wave form: always where the line
 // has one -- FP64 waves beat the dense transforms with FP32 or BF16 operands
-// too, which also need more iterations (solves, dense -> waves: 1024 x 1024
-// unknowns in FP64 589 -> 356 us; 225 x 145 in FP32 231 -> 120 us; 24 ragged
-// channels in FP32 586 -> 325 us; the 512-member ensemble with BF16 corrections
-// 3536 -> 3164 us) -- except for BF16 operands throughout, whose rounding is
-// what the caller asks for.
+// too, which also need more iterations -- except for BF16 operands throughout,
+// whose rounding is what the caller asks for.  Solves, dense -> waves, us:
+//   128 x 128 elements, order 8, FP64                     589 -> 334
+//   45 x 29, order 5, FP32                                235 -> 109
+//   512-member ensemble, BF16 corrections                3577 -> 3000
+//   256 x 256, order 8, FP64 / FP32 / BF16 corrections   2626 / 2507 / 1692 -> 1010
+//   256 x 16, order 2, one wall, FP64 / FP32              145 / 227 -> 135
+//   129 x 3, order 8, FP64                                196 -> 117
+//   64 x 3, order 2, FP64 / FP32                           89 / 150 -> 93 / 87
+// Dense is ahead where the larger residual of one application (wave_host.h)
+// costs a second iteration: order 8 and white right-hand sides, 39 x 10 elements
+// 162 -> 207, 200 x 3 238 -> 264, 256 x 16 with one wall 283 -> 385; where it does
+// not (160 x 16, 200 x 64) 224 -> 133, 299 -> 175.  That depends on the data, so no
+// rule on sizes has it.
 bool fdm_wave(const se_op* op, int prec) { return op->fdm->wave && prec != FDM_BF16; }
 
 }  // namespace

@@ -6,7 +6,8 @@
 // 5 to 19 us, whatever the size: 14 us at 1024 unknowns (p = 4), 20 us at
 // 36 672 (p = 6), 36 us at 1 048 576 (p = 8).  Here every workgroup owns a tile
 // of elements for the whole solve and the workgroups meet at grid-wide sums:
-// 5.3, 8.2 and 17.9 us per iteration at those sizes.
+// 5.2, 8.3 and 18 us per iteration at those sizes, beside 15 to 40 us for the
+// launch, the start and the check.
 //   * p of the tile stays in LDS, r, and where they fit x and the inverse
 //     diagonal, in registers.  A tile holds all nodes of its elements; a node
 //     on an edge is held by every tile around it, with the same value.
@@ -583,7 +584,14 @@ size_t grid_lds(int N, int tx, int ty, int T, int G) {
 // length and waves per SIMD; the weights are fits to measured iterations, and
 // the tiles they pick are within 2% of the best of those tried (at 32 x 32,
 // p = 6: 2 x 16 elements 6.69 ms, 4 x 8 6.64, 4 x 4 6.89, 2 x 4 7.35, 8 x 8 8.76;
-// at 8 x 8, p = 4: one workgroup 0.54 ms, two 0.59, four 0.60).
+// at 8 x 8, p = 4: one workgroup 0.54 ms, two 0.59, four 0.60).  Elsewhere they
+// are untried; what they pick beats the launches everywhere measured (ms, a
+// solve): 60 x 60 p 8 46.6 -> 22.4, 100 x 100 p 2 / 3 / 4 / 5 / 7 8.3 -> 4.4 /
+// 18.3 -> 10.5 / 28.8 -> 13.9 / 43.3 -> 21.2 / 72.1 -> 53.1, 150 x 2 p 6 45.6 -> 18.8,
+// 30 x 30 p 4 with 4 iterations 0.28 -> 0.07.  The most a tile takes is 64 elements
+// at p = 8, 72 at p = 7, 82 at p = 6: above 128 x 128 elements of p = 8 on 256 CUs
+// no tiling fits and the solve is launches again (45 us an iteration at
+// 128 x 132).
 bool grid_shape(const se_mesh* m, int cu, GridShape& best) {
     const int N = m->N, N1 = N + 1;
     double cost = HUGE_VAL;
