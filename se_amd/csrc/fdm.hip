@@ -1899,6 +1899,7 @@ int fdm_plan_solve(FdmPlan* pl, const double* const* d_f, double* const* d_x, co
             }
         }
     } else {
+        pl->desc_ok = false;  // until the new ones are up
         {
             int rc = pl->d_states.alloc(sizeof(CgState) * std::max(count, 1));
             if (rc) return rc;
