@@ -732,17 +732,14 @@ int pcg_grid(se_op* op, const double* d_f, double* d_x, const se_solve_opts& o, 
     // two regions of slots: a solve uses one and its workgroups empty theirs
     // in the other for the next solve
     constexpr size_t region = 3 * kSums * kSlots;
-    if (!op->grid_slots.ptr) {
-        int rc = op->grid_slots.alloc(2 * region * sizeof(u64));
-        if (rc) return rc;
-        op->grid_dirty = true;
+    // (memory too short for this form is enough for the other)
+    if (op->grid_slots.alloc(2 * region * sizeof(u64)) != SE_OK ||
+        op->grid_work.alloc(sizeof(double) * sh.G * ((size_t)kEdge + (size_t)grid_cells(m->N) * sh.T)) != SE_OK) {
+        (void)hipGetLastError();
+        return SE_OK;
     }
     if (op->grid_dirty) SE_HIP(hipMemsetAsync(op->grid_slots.ptr, 0xff, 2 * region * sizeof(u64), s));
     op->grid_dirty = true;  // until this solve has ended well
-    {
-        int rc = op->grid_work.alloc(sizeof(double) * sh.G * ((size_t)kEdge + (size_t)grid_cells(m->N) * sh.T));
-        if (rc) return rc;
-    }
     CgState* hs = (CgState*)op->h_state;  // pinned: the kernel writes its outcome there
     *hs = CgState{};
     GridArgs a;

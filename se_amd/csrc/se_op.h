@@ -34,7 +34,7 @@ struct se_op {
     hipGraphExec_t graph_exec = nullptr;
     int graph_iters = 0;
     se::DevBuf grid_slots, grid_work;        // one-launch solve (pcg_grid.hip): sum slots, work
-    bool grid_dirty = false;                 // they need clearing first
+    bool grid_dirty = true;                  // the slots need clearing first
     int grid_turn = 0;                       // the region the next solve uses
     int grid_tile[3] = {0, 0, 0};            // its tile's elements and threads (0: not chosen, -1: none fits)
     hipGraphExec_t graph_exec_lo = nullptr;
