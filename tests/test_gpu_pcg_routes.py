@@ -11,7 +11,7 @@ import se_amd
 
 pytestmark = pytest.mark.gpu
 
-PER, XPER, NONE = (1, 1), (1, 0), (0, 0)
+XPER = (1, 0)
 
 
 def problem(ctx, nEls, N, per=XPER, bc=(1, 1, 0, 0), seed=0):
